@@ -13,8 +13,9 @@
 //   * row_ptr is the running nnz count (:136).
 //
 // Two launches per call: `classify` (one workgroup per block and sequence)
-// packs words and counts bits; `compact` (one workgroup per sequence) scans
-// the block classes and scatters the CSR arrays and MIXED payload.  A tree
+// packs words and counts bits; `place` (up to kPlaceGroups workgroups per
+// sequence, more for very many blocks) ranks a run of blocks from the block
+// classes before it and writes their CSR entries and MIXED payload.  A tree
 // whose packed words fit in LDS (at most kSmallBlocks blocks and
 // kSmallWords words) takes one launch instead: `build_small` packs,
 // classifies and compacts a sequence in one workgroup, and `build_tree`
@@ -22,6 +23,8 @@
 // place of the block-wide scan.
 
 #include <stdlib.h>
+
+#include <algorithm>
 
 #include "tsfa_internal.h"
 
@@ -39,6 +42,7 @@ using meta::meta_geom;
 constexpr int kSmallBlocks = 256;
 constexpr int kSmallWords = 8192;  // 32 KB of packed words in LDS
 constexpr int kTreeBlocks = 64;    // one wave's lanes
+constexpr int kPlaceGroups = 512;  // workgroups per sequence of the place kernel
 
 // Nonzero bytes of x (4 mask bytes, first byte lowest) as bits 0-3: the
 // high bit of each byte of (x & 0x7f7f7f7f) + 0x7f7f7f7f | x is set iff the
@@ -116,7 +120,7 @@ __device__ inline int8_t block_class(const MetaGeom& g, int qb, int tb, int ones
 
 __global__ __launch_bounds__(kMetaThreads) void classify_kernel(
     const uint8_t* __restrict__ mask, int64_t seq_stride, int64_t row_stride, MetaGeom g,
-    int8_t* __restrict__ cls, int32_t* __restrict__ words) {
+    int8_t* __restrict__ cls, int64_t cls_stride, int32_t* __restrict__ words) {
   const int blk = blockIdx.x;  // qb * ntb + tb
   const int seq = blockIdx.y;
   const int qb = blk / g.ntb, tb = blk - qb * g.ntb;
@@ -136,7 +140,7 @@ __global__ __launch_bounds__(kMetaThreads) void classify_kernel(
   if (threadIdx.x == 0) {
     int total = 0;
     for (int i = 0; i < kMetaThreads / 64; ++i) total += red[i];
-    cls[(int64_t)seq * g.cap + blk] = block_class(g, qb, tb, total);
+    cls[seq * cls_stride + blk] = block_class(g, qb, tb, total);
   }
 }
 
@@ -163,7 +167,7 @@ __device__ inline void scan2(int a, int b, int* ex_a, int* ex_b, int* tot_a, int
 }
 
 // CSR scatter of sequence seq from its block classes c[], packed words
-// wsrc[] and rank scratch sr[] (global memory, or LDS for build_small).
+// wsrc[] and rank scratch sr[] (LDS), by one workgroup.
 __device__ inline void compact_seq(const MetaGeom& g, int seq, const int8_t* c, const int32_t* wsrc, int32_t* sr,
                                    int32_t* __restrict__ row_ptr, int32_t* __restrict__ col_idx,
                                    int8_t* __restrict__ blk_type, int32_t* __restrict__ payload,
@@ -216,19 +220,106 @@ __device__ inline void compact_seq(const MetaGeom& g, int seq, const int8_t* c, 
   }
 }
 
-__global__ __launch_bounds__(kMetaThreads) void compact_kernel(
-    MetaGeom g, const int8_t* __restrict__ cls, const int32_t* __restrict__ words,
-    int32_t* __restrict__ src_of_rank, int32_t* __restrict__ row_ptr, int32_t* __restrict__ col_idx,
-    int8_t* __restrict__ blk_type, int32_t* __restrict__ payload, int32_t* __restrict__ offset,
-    int32_t* __restrict__ counts) {
-  const int seq = blockIdx.x;
+// Second launch of the general builder: workgroup x of a sequence owns the
+// blocks [x * per, x * per + per), per <= kMetaThreads.  It counts the present
+// and the MIXED blocks before its own in the classes (16 blocks per load; rows
+// of cls are 16-byte aligned, cls_stride apart), ranks its own with one scan
+// and writes their CSR entries and payload.  One workgroup per sequence doing
+// all of it was bound by its own payload copy: 32768 words of a 1024-token
+// tree at 64 x 64 took 128 dependent load-store rounds of 256 threads, 36 us
+// (15 us when no other kernel ran between); spread over 256 workgroups 5.0 us.
+__global__ __launch_bounds__(kMetaThreads) void place_kernel(
+    MetaGeom g, int per, const int8_t* __restrict__ cls, int64_t cls_stride, const int32_t* __restrict__ words,
+    int32_t* __restrict__ row_ptr, int32_t* __restrict__ col_idx, int8_t* __restrict__ blk_type,
+    int32_t* __restrict__ payload, int32_t* __restrict__ offset, int32_t* __restrict__ counts) {
+  __shared__ int red[2 * (kMetaThreads / 64)];
+  __shared__ int s_src[kMetaThreads];  // MIXED rank within the run -> block within the run
+  const int seq = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t nb = g.cap;
-  compact_seq(g, seq, cls + seq * nb, words + seq * nb * g.words, src_of_rank + seq * nb, row_ptr, col_idx,
-              blk_type, payload, offset, counts);
+  const int64_t b0 = (int64_t)blockIdx.x * per;
+  const int n = (int)min((int64_t)per, nb - b0);  // 0 only for an empty mask
+  const int8_t* c = cls + seq * cls_stride;
+
+  // classes 0 / 1 / 2 per byte: present = bit 0 or bit 1, MIXED = bit 1
+  int nz = 0, mx = 0;
+  auto count = [&](uint32_t x) {
+    nz += __popc((x | (x >> 1)) & 0x01010101u);
+    mx += __popc(x & 0x02020202u);
+  };
+  const int64_t n16 = b0 >> 4;
+  const uint4* c16 = reinterpret_cast<const uint4*>(c);
+  for (int64_t i = tid; i < n16; i += kMetaThreads) {
+    const uint4 x = c16[i];
+    count(x.x);
+    count(x.y);
+    count(x.z);
+    count(x.w);
+  }
+  if (tid < (int)(b0 & 15)) count((uint32_t)(uint8_t)c[(n16 << 4) + tid]);
+  const int8_t k = tid < n ? c[b0 + tid] : (int8_t)kZero;
+  for (int off = 32; off > 0; off >>= 1) {
+    nz += __shfl_xor(nz, off);
+    mx += __shfl_xor(mx, off);
+  }
+  // this thread's block among its wave's present / MIXED blocks
+  const uint64_t bnz = __ballot(k != kZero), bmx = __ballot(k == kMixed), below = (1ull << lane) - 1;
+  int rank = __popcll(bnz & below), mrank = __popcll(bmx & below);
+  if (lane == 0) {
+    red[2 * wave] = nz;
+    red[2 * wave + 1] = mx;
+  }
+  __shared__ int own[2 * (kMetaThreads / 64)];
+  if (lane == 0) {
+    own[2 * wave] = __popcll(bnz);
+    own[2 * wave + 1] = __popcll(bmx);
+  }
+  __syncthreads();
+  int nz_base = 0, mx_base = 0, run_nz = 0, run_mx = 0;
+#pragma unroll
+  for (int w = 0; w < kMetaThreads / 64; ++w) {
+    nz_base += red[2 * w];
+    mx_base += red[2 * w + 1];
+    if (w < wave) {
+      rank += own[2 * w];
+      mrank += own[2 * w + 1];
+    }
+    run_nz += own[2 * w];
+    run_mx += own[2 * w + 1];
+  }
+  rank += nz_base;
+
+  int32_t* rp = row_ptr + (int64_t)seq * (g.nqb + 1);
+  if (tid < n) {
+    const int64_t i = b0 + tid;
+    const int qb = (int)(i / g.ntb), tb = (int)(i - (int64_t)qb * g.ntb);
+    if (tb == 0) rp[qb] = rank;
+    if (k != kZero) {
+      col_idx[seq * nb + rank] = tb;
+      blk_type[seq * nb + rank] = (k == kFull) ? TSFA_FULL_BLOCK : TSFA_MIXED_BLOCK;
+      offset[seq * nb + rank] = (k == kMixed) ? (mx_base + mrank) * g.words : 0;
+      if (k == kMixed) s_src[mrank] = tid;
+    }
+  }
+  if (b0 + n >= nb && tid == 0) {
+    rp[g.nqb] = nz_base + run_nz;
+    counts[2 * seq] = nz_base + run_nz;
+    counts[2 * seq + 1] = mx_base + run_mx;
+  }
+  __syncthreads();
+  const int32_t* wsrc = words + (seq * nb + b0) * g.words;
+  int32_t* pl = payload + (seq * nb + mx_base) * g.words;
+  // one wave per MIXED block, or the whole workgroup when there are few
+  const int step = run_mx >= kMetaThreads / 64 ? 64 : kMetaThreads;
+  for (int r = step == 64 ? wave : 0; r < run_mx; r += kMetaThreads / step) {
+    const int32_t* src = wsrc + (int64_t)s_src[r] * g.words;
+    int32_t* dst = pl + (int64_t)r * g.words;
+    for (int wi = step == 64 ? lane : tid; wi < g.words; wi += step) dst[wi] = src[wi];
+  }
 }
 
 // One workgroup per sequence: packed words and block bit counts in LDS,
-// classes, then the same scatter as compact_kernel.
+// classes, then the scatter.
 __global__ __launch_bounds__(kMetaThreads) void build_small_kernel(
     const uint8_t* __restrict__ mask, int64_t seq_stride, int64_t row_stride, MetaGeom g,
     int32_t* __restrict__ row_ptr, int32_t* __restrict__ col_idx, int8_t* __restrict__ blk_type,
@@ -362,11 +453,11 @@ extern "C" int tsfa_meta_build(const uint8_t* mask, int64_t mask_seq_stride, int
                     offset == nullptr))
     return TSFA_ERR_INVALID_ARGUMENT;
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
-  const size_t nb = (size_t)n_seq * g.cap;
+  // workspace: block classes (a 16-byte aligned row per sequence), packed words
+  const int64_t cls_stride = meta::class_stride(g);
   int8_t* cls = static_cast<int8_t*>(workspace);
-  int32_t* words = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + align256(nb));
-  int32_t* src_of_rank =
-      reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + align256(nb) + align256(nb * g.words * 4));
+  int32_t* words =
+      reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + align256((size_t)n_seq * cls_stride));
   const bool small = g.cap > 0 && g.cap <= kSmallBlocks && g.cap * g.words <= kSmallWords &&
                      config().meta_small != 0;  // TSFA_META_SMALL=0: always two launches
   if (small && g.cap <= kTreeBlocks) {
@@ -395,11 +486,17 @@ extern "C" int tsfa_meta_build(const uint8_t* mask, int64_t mask_seq_stride, int
   if (g.cap > 0) {
     if (g.cap > INT32_MAX) return TSFA_ERR_UNSUPPORTED;
     hipLaunchKernelGGL(classify_kernel, dim3((unsigned)g.cap, (unsigned)n_seq), dim3(kMetaThreads), 0, stream,
-                       mask, mask_seq_stride, mask_row_stride, g, cls, words);
+                       mask, mask_seq_stride, mask_row_stride, g, cls, cls_stride, words);
     if (hipGetLastError() != hipSuccess) return TSFA_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL(compact_kernel, dim3((unsigned)n_seq), dim3(kMetaThreads), 0, stream, g, cls, words,
-                     src_of_rank, row_ptr, col_idx, blk_type, payload, offset, counts);
+  // a block per workgroup while that leaves at most kPlaceGroups of them, and
+  // never more blocks than threads
+  const int64_t groups = std::max<int64_t>(1, std::max((g.cap + kMetaThreads - 1) / kMetaThreads,
+                                                       std::min<int64_t>(g.cap, kPlaceGroups)));
+  const int per = (int)std::max<int64_t>(1, (g.cap + groups - 1) / groups);
+  const unsigned grid = (unsigned)std::max<int64_t>(1, (g.cap + per - 1) / per);
+  hipLaunchKernelGGL(place_kernel, dim3(grid, (unsigned)n_seq), dim3(kMetaThreads), 0, stream, g, per, cls,
+                     cls_stride, words, row_ptr, col_idx, blk_type, payload, offset, counts);
   if (hipGetLastError() != hipSuccess) return TSFA_ERR_LAUNCH;
   return TSFA_OK;
 }

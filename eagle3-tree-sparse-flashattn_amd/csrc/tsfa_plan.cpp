@@ -422,8 +422,7 @@ extern "C" size_t tsfa_meta_workspace_bytes(int n_seq, int q_len, int block_m, i
   if (tsfa_meta_check_args(n_seq, q_len, block_m, block_n) != TSFA_OK) return 0;
   meta::MetaGeom g;
   meta::meta_geom(q_len, block_m, block_n, &g);
-  const size_t nb = (size_t)n_seq * g.cap;
-  return align256(nb) + align256(nb * g.words * 4) + align256(nb * 4);
+  return align256((size_t)n_seq * meta::class_stride(g)) + align256((size_t)n_seq * g.cap * g.words * 4);
 }
 
 // The tree metadata of n_seq masks on the host, in tsfa_meta_build's layout

@@ -142,6 +142,11 @@ struct MetaGeom {
 
 bool meta_geom(int q_len, int block_m, int block_n, MetaGeom* g);
 
+// Bytes between the block classes of two sequences in the builder's
+// workspace: rows the place kernel reads 16 classes at a time start 16-byte
+// aligned (fewer than 16 blocks are read one by one).
+inline int64_t class_stride(const MetaGeom& g) { return g.cap < 16 ? g.cap : (g.cap + 15) / 16 * 16; }
+
 }  // namespace meta
 
 }  // namespace tsfa

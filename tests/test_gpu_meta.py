@@ -70,6 +70,21 @@ def test_sweep(q_len, bm, bn, kind, seed, path, monkeypatch):
     assert_meta_equal(meta, mo.build_metadata(m, 11, bm, bn))
 
 
+# the general builder's second launch at its run lengths (one block per
+# workgroup, runs of several, more runs than kPlaceGroups) and class counts
+# off 16, and word loads at odd row strides, cut rows and sliced masks
+@pytest.mark.parametrize("q_len,bm,bn,n_seq", [(61, 64, 64, 3), (95, 32, 32, 1), (300, 16, 16, 3), (515, 16, 16, 1),
+                                               (777, 64, 64, 2), (720, 2, 2, 1), (1030, 64, 128, 1)])
+def test_runs_of_blocks_and_cut_rows(q_len, bm, bn, n_seq):
+    rng = np.random.default_rng(q_len)
+    wide = torch.from_numpy(rng.random((n_seq, q_len, q_len + 5)) < 0.02).cuda()
+    masks = wide[:, :, 3:3 + q_len]
+    masks[:, : 2 * bm, : 2 * bn] = True
+    got = tsf.prepare_tree_sparse_metadata_batched(masks, 11, bm, bn)
+    for b in range(n_seq):
+        assert_meta_equal(got.sequence(b), mo.build_metadata(masks[b].cpu().numpy(), 11, bm, bn))
+
+
 def test_nonbool_masks():
     vals = torch.tensor([[0.0, float("nan"), -1.5], [2.0, 0.0, 0.0], [0.0, 0.0, 1e-30]])
     for m in (vals, vals.to(torch.float16), (vals != 0).to(torch.int32) * 7):
