@@ -1676,11 +1676,13 @@ int launch_all(const SplitArgs& sa_in, const CombineArgs& ca, const Plan& p, con
 // and the 4 rows x 4 chunks of a transposing V^T read spread over the LDS
 // banks (a 512-byte row stride maps every row to the same banks; XOR with
 // k & 15 on V only permutes chunks inside their group of 4, which measured
-// bank conflicts on half of the LDS cycles).  The fp32 instances keep
-// rows unswizzled: their 4-byte operand reads then use immediate offsets
-// (with the XOR, one address register per read spills the head_dim 256
-// instance), and their 32x32x2 MFMAs, at 1/16 of the 16-bit rate, bound
-// the loop anyway.
+// bank conflicts on half of the LDS cycles).  The fp32 instances read 16
+// bytes per lane too, each read feeding four 32x32x2 MFMAs (the order of the
+// contraction and of O's columns over the MFMAs is free): K's chunks are
+// swizzled as above, a V row is read whole by the 32 lanes of a half-wave
+// and needs none.  They are bound by the fp32 matrix rate; with one word per
+// lane of unswizzled rows every K read was a 32-way bank conflict (the 8B
+// decode shape in fp32: 103.5 -> 58.3 us per call).
 struct GenArgs {
   const void* q;
   const void* k;
@@ -1739,9 +1741,13 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
   constexpr int NSTG = kGenStages(SB);
   constexpr int LPW = SB / 1024 / NW;  // 1 KB loads per wave per unit
   constexpr int DT = D / 32 / DS;      // O d-tiles of a wave
-  constexpr int KS = F32 ? D / 2 : D / 16;  // k-steps of S^T
+  constexpr int KS = F32 ? D / 8 : D / 16;  // K reads of S^T: one MFMA each, fp32 four
   // chunk c of row k at c ^ (k & SWZ) in K, c ^ ((k & SWV) << 2) in V
-  constexpr int SWZ = F32 ? 0 : 15, SWV = F32 ? 0 : 3;
+  constexpr int SWZ = 15, SWV = F32 ? 0 : 3;
+  // fp32: words of a V row per lane and read; register e of read h is column
+  // 128h + EPL*ln + e of the row, so O's d-tile dt holds the columns
+  // 128*(dt/EPL) + EPL*m + dt%EPL (m = 0..31)
+  constexpr int EPL = D / 32 < 4 ? D / 32 : 4;
   static_assert(CPR >= 16 && LPW >= 1 && LPW * (NSTG - 2) < 64 && SB % (1024 * NW) == 0, "generic ring");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
@@ -1765,16 +1771,15 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
   const T* qrow = static_cast<const T*>(a.q) + b * a.sqb + (int64_t)(kvh * G + g) * a.sqh + (int64_t)t * a.sqm;
 
   // Q^T operand: 16-bit, lane (ln, lh) holds d = 16kk + 8lh + [0, 8) of its
-  // row; fp32, d = 2kk + lh (16-byte loads, the lane keeps its two words of
-  // each).  Q is negated for a negative scale.
-  typedef typename std::conditional<F32, float, i16x8>::type QF;
+  // row; fp32, d = 8kk + 4lh + [0, 4), one per MFMA.  Q is negated for a
+  // negative scale.
+  typedef typename std::conditional<F32, f32x4, i16x8>::type QF;
   QF qf[KS];
 #pragma unroll
-  for (int kk = 0; kk < KS; kk += (F32 ? 2 : 1)) {
+  for (int kk = 0; kk < KS; ++kk) {
     if constexpr (F32) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(qrow + 2 * kk);
-      qf[kk] = a.neg_q ? -(lh ? x[1] : x[0]) : (lh ? x[1] : x[0]);
-      qf[kk + 1] = a.neg_q ? -(lh ? x[3] : x[2]) : (lh ? x[3] : x[2]);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(qrow + 8 * kk + 4 * lh);
+      qf[kk] = a.neg_q ? -x : x;
     } else {
       qf[kk] = *reinterpret_cast<const i16x8*>(qrow + 16 * kk + 8 * lh) ^ (short)(a.neg_q ? 0x8000 : 0);
     }
@@ -1892,24 +1897,17 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
     f32x16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
-    constexpr int KA = F32 ? 8 : 4;
-    typedef typename std::conditional<F32, float, i16x8>::type KF;
-    KF kf[KS];
-    auto rk = [&](int kk) {
-      if constexpr (F32) {
-        const int wd = 2 * kk + lh;  // word of the row
-        kf[kk] = *reinterpret_cast<const float*>(kt + swz(ln, wd >> 2) + (wd & 3) * 4);
-      } else {
-        kf[kk] = *reinterpret_cast<const i16x8*>(kt + swz(ln, 2 * kk + lh));
-      }
-    };
+    constexpr int KA = F32 ? 2 : 4;
+    QF kf[KS];
+    auto rk = [&](int kk) { kf[kk] = *reinterpret_cast<const QF*>(kt + swz(ln, 2 * kk + lh)); };
 #pragma unroll
     for (int kk = 0; kk < KA; ++kk) rk(kk);
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk) {
       if (kk + KA < KS) rk(kk + KA);
       if constexpr (F32) {
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[kk], qf[kk], s, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[kk][e], qf[kk][e], s, 0, 0, 0);
       } else {
         s = Mma<T>::run(bit_cast<typename Mma<T>::vec8>(kf[kk]), bit_cast<typename Mma<T>::vec8>(qf[kk]), s);
       }
@@ -1960,16 +1958,27 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
     // O^T += V^T P^T, P rounded to the input dtype (tree_sparse_flashattn.py:278)
     if constexpr (F32) {
       // k-step i: keys 8*(i/4) + 4*k + i%4 (k = 0, 1), lane (ln, lh) gives its
-      // element i of P^T and V[key 8*(i/4) + 4*lh + i%4][32*dt + ln] of V^T
+      // element i of P^T and EPL words of V's row 8*(i/4) + 4*lh + i%4, one
+      // per d-tile (V read VA reads ahead)
+      typedef float VF __attribute__((ext_vector_type(EPL)));
+      constexpr int NH = DT / EPL, VA = 2;
+      VF vf[16 * NH];
+      auto rv = [&](int x) {
+        const int i = x / NH, key = 8 * (i >> 2) + 4 * lh + (i & 3);
+        vf[x] = *reinterpret_cast<const VF*>(vt + key * ROWB + 512 * (x % NH) + 4 * EPL * ln);
+      };
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
+      for (int x = 0; x < VA; ++x) rv(x);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int key = 8 * (i >> 2) + 4 * lh + (i & 3);
-          const int wd = 32 * (dh * DT + dt) + ln;
-          const float vv = *reinterpret_cast<const float*>(vt + swv(key, wd >> 2) + (wd & 3) * 4);
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, p[i], o[dt], 0, 0, 0);
+      for (int x = 0; x < 16 * NH; ++x) {
+        if (x + VA < 16 * NH) rv(x + VA);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+          const int dt = EPL * (x % NH) + e;
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[x][e], p[x / NH], o[dt], 0, 0, 0);
         }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     } else {
       typedef typename Mma<T>::vec8 V8;
       V8 pb[2];
@@ -2005,24 +2014,46 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
     }
   }
 
+  // The lane's O row: 4 consecutive columns per store, w scaling them.
+  // 16-bit: columns 32dt + 8j + 4lh + [0, 4) of the wave's part are elements
+  // 4j.. of d-tile dt; fp32 (d-tiles interleaved): columns 128h + EPL*(8q +
+  // 4lh) + [0, 4*EPL) are elements 4q.. of d-tiles EPL*h.., tile fastest.
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  auto store_row = [&](T* dst, float w) {
+    if constexpr (F32) {
+#pragma unroll
+      for (int h = 0; h < DT / EPL; ++h)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int y = 0; y < EPL; ++y) {
+            T4 x;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int c = 4 * y + e;  // column after 128h + EPL*(8q + 4lh)
+              x[e] = o[EPL * h + c % EPL][4 * q + c / EPL] * w;
+            }
+            *reinterpret_cast<T4*>(dst + 128 * h + EPL * (8 * q + 4 * lh) + 4 * y) = x;
+          }
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *reinterpret_cast<T4*>(dst + 32 * (dh * DT + dt) + 8 * j + 4 * lh) =
+              T4{(T)(o[dt][4 * j] * w), (T)(o[dt][4 * j + 1] * w), (T)(o[dt][4 * j + 2] * w),
+                 (T)(o[dt][4 * j + 3] * w)};
+    }
+  };
+
   const float lt = pair_sum(l_run);
   if (a.direct) {
     // a one-split plan writes the lane's row of O (token t, head kvh*G + g)
     // in the input dtype: one rounding of the fp32 result; a row that saw no
     // key gets NaN (0/0, as the reference and the combine give)
-    if (row_ok) {
-      typedef T T4 __attribute__((ext_vector_type(4)));
-      const float inv_o = lt > 0.f ? 1.f / lt : __builtin_nanf("");
-      T* dst = static_cast<T*>(a.out) + b * a.sob + (int64_t)(kvh * G + g) * a.soh + (int64_t)t * a.som +
-               32 * DT * dh;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          *reinterpret_cast<T4*>(dst + 32 * dt + 8 * j + 4 * lh) =
-              T4{(T)(o[dt][4 * j] * inv_o), (T)(o[dt][4 * j + 1] * inv_o), (T)(o[dt][4 * j + 2] * inv_o),
-                 (T)(o[dt][4 * j + 3] * inv_o)};
-    }
+    if (row_ok)
+      store_row(static_cast<T*>(a.out) + b * a.sob + (int64_t)(kvh * G + g) * a.soh + (int64_t)t * a.som,
+                lt > 0.f ? 1.f / lt : __builtin_nanf(""));
     return;
   }
   // partial of the lane's row: O / l in the input dtype (as the split
@@ -2032,15 +2063,7 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
   const int64_t prow = ((int64_t)bk * a.n_slots + slot) * TG + r;
   if (row_ok) {
-    typedef T T4 __attribute__((ext_vector_type(4)));
-    T* dst = static_cast<T*>(a.ws_o) + prow * D + 32 * DT * dh;  // the wave's columns
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        *reinterpret_cast<T4*>(dst + 32 * dt + 8 * j + 4 * lh) =
-            T4{(T)(o[dt][4 * j] * inv), (T)(o[dt][4 * j + 1] * inv), (T)(o[dt][4 * j + 2] * inv),
-               (T)(o[dt][4 * j + 3] * inv)};
+    store_row(static_cast<T*>(a.ws_o) + prow * D, inv);
     if (lh == 0 && dh == 0) a.ws_ml[prow] = make_float2(m_run, lt);
   }
 }
