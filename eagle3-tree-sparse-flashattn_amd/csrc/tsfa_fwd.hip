@@ -1899,7 +1899,11 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
     constexpr int KA = F32 ? 2 : 4;
     QF kf[KS];
-    auto rk = [&](int kk) { kf[kk] = *reinterpret_cast<const QF*>(kt + swz(ln, 2 * kk + lh)); };
+    // fp32: read offsets formed anew each unit (hoisted out of the loop they
+    // spill the head_dim 256 instance)
+    int kr = ln;
+    if constexpr (F32) asm volatile("" : "+v"(kr));
+    auto rk = [&](int kk) { kf[kk] = *reinterpret_cast<const QF*>(kt + swz(kr, 2 * kk + lh)); };
 #pragma unroll
     for (int kk = 0; kk < KA; ++kk) rk(kk);
 #pragma unroll
