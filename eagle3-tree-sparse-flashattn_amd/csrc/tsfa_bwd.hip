@@ -52,6 +52,7 @@
 #include <atomic>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "tsfa_internal.h"
@@ -103,6 +104,15 @@ template <int N> __device__ inline void vm_wait() {
 }
 __device__ inline void sync_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ inline uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const TSFA_LDS void*)p; }
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// LDS reads at addr + off (off: the instruction's immediate offset).
+template <typename V> __device__ inline V lds_ld(uint32_t addr, int off = 0) {
+  return *(const TSFA_LDS V*)((const TSFA_LDS char*)(uintptr_t)addr + off);
+}
+__device__ inline i16x4 lds_tr(uint32_t addr, int off) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((TSFA_LDS i16x4*)((TSFA_LDS char*)(uintptr_t)addr + off));
+}
+__device__ inline void fence_order() { __builtin_amdgcn_sched_barrier(0); }
 template <typename V, typename U> __device__ inline V bit_cast(U u) { return __builtin_bit_cast(V, u); }
 
 struct BwdArgs {
@@ -113,7 +123,7 @@ struct BwdArgs {
   void* dk;
   void* dv;
   float* dq_acc;            // [B*Hkv][D][n_tiles*32] fp32 (d-major: a wave's atomics cover whole lines)
-  const float2* rowstat;    // [B*Hkv][n_tiles*32] (log2 LSE, Dv)
+  const float* rowstat;     // [B*Hkv][n_tiles][2][32]: log2 LSE, then Dv, of the tile's rows
   const uint32_t* vis;      // [n_trees][n_tiles][n_tkeys] visibility words of tree keys
   int64_t sqb, sqh, sqm, skb, skh, skn, svb, svh, svn, sdob, sdoh, sdom, sdkb, sdkh, sdkn, sdvb, sdvh, sdvn;
   int64_t vis_tree_stride;  // 0: one tree for the batch
@@ -123,6 +133,8 @@ struct BwdArgs {
   int n_tiles, n_pb, n_tb, n_tkeys;
   int n_items, items_per_xcd;
   uint32_t group_magic;     // floor(2^32 / group) + 1 (group > 1): R / group = umulhi(R, magic) for R < 2^21
+  int tile_fast;            // whole Q / dO tiles at a scalar base + fixed 32-bit lane offsets (group divides 32)
+  int key_fast;             // the same for whole 32-key K / V units
   // row-parallel dQ kernel
   void* dq;                 // dq_direct: the kernel writes sm_scale * dQ here (one split per chunk)
   int64_t sdqb, sdqh, sdqm;
@@ -134,9 +146,9 @@ struct BwdArgs {
 
 template <int D> constexpr size_t kv_lds_bytes() {
   // K block | V block | 2 groups x kBufs x (Q tile, dO tile) | 2 x kBufs x 32 row stats |
-  // 2 x kBufs x 128 mask words | 64 bytes of dummy load targets
+  // 2 x kBufs x 128 mask words
   return 2 * (size_t)kBlockKeys * D * 2 + 2 * 2 * kBufs * (size_t)kTileRows * D * 2 + 2 * kBufs * kTileRows * 8 +
-         2 * kBufs * kBlockKeys * 4 + 64;
+         2 * kBufs * kBlockKeys * 4;
 }
 
 // Workgroup = 8 waves: key group kg = wave & 3 owns keys key0 + 32kg + [0, 32);
@@ -144,6 +156,18 @@ template <int D> constexpr size_t kv_lds_bytes() {
 // wave of each row group, so one wave's softmax-like VALU work and LDS waits
 // overlap the other's MFMAs.  Both groups accumulate dK^T / dV^T of the same
 // keys; group 1 hands its sums to group 0 through LDS at the end.
+//
+// What bounds it: latency, not a pipe (MFMA busy 36 % and 8.6 VALU per MFMA
+// at the 1024-token tree behind 16k keys when the step ran S and dP, then
+// all of the softmax, then dV and dK: both waves of a SIMD sat in the same
+// phase).  A tile now runs four MFMA groups with the VALU work between the
+// MFMAs of the next group that does not need it -- S; dP with P's
+// exponentials; dV with dS; dK -- and operands read RA / VA MFMAs ahead, in a
+// fixed order.  Blocks whose 128 keys are all visible compile without the
+// mask, and whole tiles of a group that divides 32 are addressed by a scalar
+// base plus fixed lane offsets (the general path costs ~15 VALU per 1 KB
+// load): 1.53 M -> 1.27 M cycles at that shape, 243 -> 105 VALU instructions
+// per 32 MFMAs.
 template <typename T, int D>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_kv_kernel(const BwdArgs a) {
@@ -158,17 +182,15 @@ void bwd_kv_kernel(const BwdArgs a) {
   constexpr int LPT = TILE_B / 1024;          // 1 KB loads per Q (or dO) tile
   constexpr int TPW = 2 * LPT / 4;            // tile loads per wave (4 waves per row group)
   constexpr int KPW = 2 * KBLK_B / 1024 / kWaves;  // K + V block loads per wave
-  constexpr int LPW = TPW + 1;                // vector-memory instructions a wave issues per tile
   static_assert(kBufs == 2, "the exchange at the end reuses the K, V and tile areas");
   static_assert(TPW >= 1 && KPW >= 1 && 2 * LPT == TPW * 4, "load split");
 
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  extern __shared__ __attribute__((aligned(256))) unsigned char smem[];  // tile bases keep bits 0-7 clear
   unsigned char* kblk = smem;
   unsigned char* vblk = kblk + KBLK_B;
   unsigned char* tiles = vblk + KBLK_B;  // group g, buffer s: Q at tiles + 2*(g*kBufs + s)*TILE_B, dO after
-  float2* rs = reinterpret_cast<float2*>(tiles + 2 * 2 * kBufs * TILE_B);          // [g][s][32]
-  uint32_t* visw = reinterpret_cast<uint32_t*>(rs + 2 * kBufs * kTileRows);        // [g][s][128]
-  unsigned char* dummy = reinterpret_cast<unsigned char*>(visw + 2 * kBufs * kBlockKeys);
+  float* rs = reinterpret_cast<float*>(tiles + 2 * 2 * kBufs * TILE_B);            // [g][s][2][32]
+  uint32_t* visw = reinterpret_cast<uint32_t*>(rs + 2 * kBufs * 2 * kTileRows);    // [g][s][128]
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -191,14 +213,13 @@ void bwd_kv_kernel(const BwdArgs a) {
   const int key_end = tree_blk ? a.kv_len : a.prefix_len;  // keys of this block: [key0, min(key0 + 128, key_end))
   const int G = a.group;
   const int TG = a.q_len * G;
-  const int TGP = a.n_tiles * kTileRows;
   const float sl2 = a.scale_log2;  // signed: exp2(s * sl2 - lse2) for either sign of sm_scale
 
   const T* kbase = static_cast<const T*>(a.k) + b * a.skb + kvh * a.skh;
   const T* vbase = static_cast<const T*>(a.v) + b * a.svb + kvh * a.svh;
   const T* qbase = static_cast<const T*>(a.q) + b * a.sqb + (int64_t)kvh * G * a.sqh;
   const T* dobase = static_cast<const T*>(a.dout) + b * a.sdob + (int64_t)kvh * G * a.sdoh;
-  const float2* rsbase = a.rowstat + (int64_t)bk * TGP;
+  const float* rsbase = a.rowstat + (int64_t)bk * a.n_tiles * (2 * kTileRows);
   const uint32_t* visbase =
       a.vis + (int64_t)b * a.vis_tree_stride + (tree_blk ? (int64_t)tkb * kBlockKeys : 0);
 
@@ -214,66 +235,67 @@ void bwd_kv_kernel(const BwdArgs a) {
     dma16(src, lds_addr((is_v ? vblk : kblk) + ul * 1024));
   }
 
-  // The tiles of row group rg: step n handles tile tile_at(2n + rg).  The key
-  // blocks of one (b, kv head) start their walk at different tiles (block kb
-  // at tile kb * n_tiles / nkb), so the dQ atomics of concurrent blocks land
-  // on different rows.
-  const int j0 = (int)((int64_t)kb * a.n_tiles / nkb);
-  auto tile_at = [&](int i) {
-    const int j = j0 + i;
-    return j >= a.n_tiles ? j - a.n_tiles : j;
-  };
+  // The tiles of row group rg: step n handles tile 2n + rg.
   const int n_steps = (a.n_tiles + 1) >> 1;
   const int my_tiles = (a.n_tiles + 1 - rg) >> 1;  // steps with a tile for this group
 
-  // Q / dO tile j -> this group's buffer s, with its row statistics and (tree
-  // blocks) the 128 keys' mask words.  Every wave issues exactly LPW loads
-  // per tile: its share of Q and dO plus one more (the row statistics for key
-  // group 0, the mask words for key group 1 of a tree block, else one lane
-  // into a dummy LDS slot), so the waits below are compile-time counts.
-  // Rows past the end repeat the last row; their statistics make P = dS = 0.
-  auto issue_tile = [&](int j, int s) {
-    unsigned char* qt = tiles + 2 * (rg * kBufs + s) * TILE_B;
+  // Q / dO tile j -> this group's buffer s, with its row statistics (key
+  // group 0) and, for tree blocks, the 128 keys' mask words (key group 1).
+  // Key groups 0 and 1 move the Q tile, 2 and 3 the dO tile.  Rows past the
+  // end repeat the last row; their statistics make P = dS = 0.
+  const bool is_do = kg >= 2;
+  const T* tbase = is_do ? dobase : qbase;
+  const int64_t tsh = is_do ? a.sdoh : a.sqh, tsm = is_do ? a.sdom : a.sqm;
+  auto load_row = [&](int i) { return ((kg & 1) * TPW + i) * RPL + lane / CPR; };
+  uint32_t toff[TPW];  // tile_fast: lane byte offsets from the tile's first token
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      const int u = kg * TPW + i;  // 0 .. 2*LPT-1: Q loads, then dO loads
-      const bool is_do = u >= LPT;
-      const int ul = is_do ? u - LPT : u;
-      const int row = ul * RPL + lane / CPR, pos = lane % CPR;
-      const int R = min(j * kTileRows + row, TG - 1);
-      const int t = G == 1 ? R : (int)__umulhi((uint32_t)R, a.group_magic);
-      const int g = R - t * G;
-      const T* src = is_do ? dobase + g * a.sdoh + (int64_t)t * a.sdom : qbase + g * a.sqh + (int64_t)t * a.sqm;
-      dma16(src + ((pos ^ swz<D>(row)) << 3), lds_addr(qt + (is_do ? TILE_B : 0) + ul * 1024));
+  for (int i = 0; i < TPW; ++i) {
+    const int row = load_row(i), t = G == 1 ? row : row / G;
+    toff[i] = (uint32_t)(((int64_t)(row - t * G) * tsh + (int64_t)t * tsm + (((lane % CPR) ^ swz<D>(row)) << 3)) * 2);
+  }
+  const int tpt = a.tile_fast ? kTileRows / G : 0;  // tokens per tile
+  auto issue_tile = [&](int j, int s) {
+    const uint32_t tl = lds_addr(tiles + 2 * (rg * kBufs + s) * TILE_B + (is_do ? TILE_B : 0) + (kg & 1) * TPW * 1024);
+    if (a.tile_fast && (j + 1) * kTileRows <= TG) {
+      const T* src = tbase + (int64_t)j * tpt * tsm;
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) dma16_s(src, toff[i], tl + i * 1024);
+    } else {
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+        const int row = load_row(i);
+        const int R = min(j * kTileRows + row, TG - 1);
+        const int t = G == 1 ? R : (int)__umulhi((uint32_t)R, a.group_magic);
+        const int g = R - t * G;
+        dma16(tbase + g * tsh + (int64_t)t * tsm + (((lane % CPR) ^ swz<D>(row)) << 3), tl + i * 1024);
+      }
     }
     if (kg == 0) {
-      if (lane < kTileRows * 8 / 16)
-        dma16_s(rsbase + j * kTileRows, 16u * lane, lds_addr(rs + (rg * kBufs + s) * kTileRows));
+      if (lane < 2 * kTileRows * 4 / 16)
+        dma16_s(rsbase + (int64_t)j * (2 * kTileRows), 16u * lane, lds_addr(rs + (rg * kBufs + s) * 2 * kTileRows));
     } else if (kg == 1 && tree_blk) {
       if (lane < kBlockKeys * 4 / 16)
         dma16_s(visbase + (int64_t)j * a.n_tkeys, 16u * lane, lds_addr(visw + (rg * kBufs + s) * kBlockKeys));
-    } else if (lane == 0) {
-      dma16_s(rsbase, 0u, lds_addr(dummy + 16 * (wave & 3)));
     }
   };
-  for (int i = 0; i < kBufs - 1 && i < my_tiles; ++i) issue_tile(tile_at(2 * i + rg), i);
+  if (my_tiles > 0) issue_tile(rg, 0);
 
   const int mykey = key0 + 32 * kg + ln;
   const bool key_ok = mykey < key_end && mykey < key0 + kBlockKeys;
+  const bool all_keys = !tree_blk && key0 + kBlockKeys <= key_end;  // every key visible to every row
 
-  // LDS offsets (bytes).  Row reads: lane (row ln, lh) reads chunk 2kk + lh.
-  // Transposed reads: lane (x = lane>>4, i = lane&15) reads 8 bytes of row
-  // 8jj + 4(x>>1) + (i>>2) (+16 per k-step) at d = dt*32 + 16(x&1) + 4(i&3);
-  // after the transpose it holds rows +[0,4) of d = dt*32 + 16(x&1) + i.
+  // LDS offsets (bytes).  Row reads: lane (row ln, lh) reads chunk 2kk + lh,
+  // at r_off0 ^ (kk << 5).  Transposed reads: lane (x = lane>>4, i = lane&15)
+  // reads 8 bytes of row 8jj + 4(x>>1) + (i>>2) (+16 per k-step) at d = dt*32
+  // + 16(x&1) + 4(i&3), i.e. at (t_off0 ^ (dt << 6) ^ (jj << 5)) + 8jj rows
+  // (8 rows on, the swizzle flips chunk bit 1); after the transpose it holds
+  // rows +[0,4) of d = dt*32 + 16(x&1) + i.
   const int vx = lane >> 4, vi = lane & 15;
-  auto r_off = [&](int kk) { return ln * ROWB + (((2 * kk + lh) ^ swz<D>(ln)) << 4); };
-  auto t_off = [&](int dt, int jj) {
-    const int r = 8 * jj + 4 * (vx >> 1) + (vi >> 2);
-    const int d = dt * 32 + 16 * (vx & 1) + 4 * (vi & 3);
-    return r * ROWB + (((d >> 3) ^ swz<D>(r)) << 4) + ((d & 7) << 1);
-  };
-  const unsigned char* kmine = kblk + 32 * kg * ROWB;
-  const unsigned char* vmine = vblk + 32 * kg * ROWB;
+  const int trow = 4 * (vx >> 1) + (vi >> 2);
+  const uint32_t r_off0 = (uint32_t)(ln * ROWB + ((lh ^ swz<D>(ln)) << 4));
+  const uint32_t t_off0 =
+      (uint32_t)(trow * ROWB + (((2 * (vx & 1) + ((vi & 3) >> 1)) ^ swz<D>(trow)) << 4) + ((vi & 1) << 3));
+  const uint32_t kmine = lds_addr(kblk + 32 * kg * ROWB);  // V: KBLK_B further
 
   f32x16 dk[DT], dv[DT];
 #pragma unroll
@@ -281,79 +303,121 @@ void bwd_kv_kernel(const BwdArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) dk[dt][i] = dv[dt][i] = 0.f;
 
-  // rows (keys) +0..3 and +8..11 of a transposed read: the two halves of
-  // one operand (jj = 0, 1; the swizzle differs between them)
-  auto tr_pair = [&](const unsigned char* base, int dt) {
-    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TSFA_LDS i16x4*)(base + t_off(dt, 0)));
-    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TSFA_LDS i16x4*)(base + t_off(dt, 1)));
-    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  // One tile from buffer s.  masked_c: tree blocks and the prefix's partial
+  // last block (P = 0 for the lane's key where its mask bit is clear).
+  auto tile_step = [&](auto masked_c, int s) {
+    constexpr bool MASKED = decltype(masked_c)::value;
+    constexpr int RA = 3;          // row-operand pairs read ahead
+    constexpr int VA = 3;          // transposed pairs read ahead
+    constexpr int EP = 16 / KSTEPS;  // P (dS) elements between two MFMAs
+    constexpr int NG = 2 * DT;     // dV (dK) MFMAs
+    static_assert(NG == KSTEPS, "one slice of P and of dS per MFMA");
+    const uint32_t qt = lds_addr(tiles + 2 * (rg * kBufs + s) * TILE_B);
+    // (read offsets formed anew each tile: hoisted out of the loop they spill)
+    uint32_t q0 = qt + r_off0, k0 = kmine + r_off0, t0 = qt + t_off0;
+    asm volatile("" : "+v"(q0), "+v"(k0), "+v"(t0));
+    const uint32_t st = lds_addr(rs + (rg * kBufs + s) * 2 * kTileRows) + 16u * lh;
+    uint32_t w = 0;
+    if constexpr (MASKED) {
+      w = key_ok ? 0xffffffffu : 0u;
+      if (tree_blk) w &= visw[(rg * kBufs + s) * kBlockKeys + 32 * kg + ln];
+      w >>= 4 * lh;
+    }
+    // S = Q K^T, dP = dO V^T: M = rows, N = keys; lane (key ln, lh) holds
+    // rows 8(i/4) + 4lh + i%4 of its key.  Operand pair x: S's k-steps, then dP's.
+    i16x8 fa[2 * KSTEPS], fb[2 * KSTEPS];
+    auto rd = [&](int x) {
+      const uint32_t c = (uint32_t)((x % KSTEPS) << 5);
+      fa[x] = lds_ld<i16x8>(q0 ^ c, x < KSTEPS ? 0 : TILE_B);
+      fb[x] = lds_ld<i16x8>(k0 ^ c, x < KSTEPS ? 0 : KBLK_B);
+    };
+    // transposed pair x: dO's NG, then Q's (one LDS copy serves both reads)
+    i16x4 tl[2 * NG], th[2 * NG];
+    auto rt = [&](int x) {
+      const int g = x % NG, dt = g >> 1, s2 = g & 1;
+      const uint32_t c = t0 ^ (uint32_t)(dt << 6);
+      const int off = (x < NG ? TILE_B : 0) + 16 * s2 * ROWB;
+      tl[x] = lds_tr(c, off);
+      th[x] = lds_tr(c ^ 32u, off + 8 * ROWB);
+    };
+    auto tr = [&](int x) { return bit_cast<V8>(__builtin_shufflevector(tl[x], th[x], 0, 1, 2, 3, 4, 5, 6, 7)); };
+    f32x4 lse4[4], dv4[4];  // statistics of the lane's rows 8q + 4lh + [0, 4)
+    f32x16 sc, dp;
+    V8 pb[2], db[2];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sc[i] = dp[i] = 0.f;
+    auto p_slice = [&](int y) {
+#pragma unroll
+      for (int i = EP * y; i < EP * (y + 1); ++i) {
+        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], sl2, -lse4[i >> 2][i & 3]));
+        if constexpr (MASKED) p = ((w >> (8 * (i >> 2) + (i & 3))) & 1u) ? p : 0.f;
+        sc[i] = p;
+        pb[i >> 3][i & 7] = (T)p;
+      }
+    };
+    auto ds_slice = [&](int y) {
+#pragma unroll
+      for (int i = EP * y; i < EP * (y + 1); ++i) db[i >> 3][i & 7] = (T)(sc[i] * (dp[i] - dv4[i >> 2][i & 3]));
+    };
+#pragma unroll
+    for (int x = 0; x < RA; ++x) rd(x);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) lse4[q] = lds_ld<f32x4>(st, 32 * q);
+    fence_order();
+#pragma unroll
+    for (int x = 0; x < KSTEPS; ++x) {
+      rd(x + RA);
+      sc = Mma<T>::run(bit_cast<V8>(fa[x]), bit_cast<V8>(fb[x]), sc);
+      fence_order();
+    }
+#pragma unroll
+    for (int x = KSTEPS; x < 2 * KSTEPS; ++x) {
+      if (x + RA < 2 * KSTEPS) rd(x + RA);
+      else rt(x + RA - 2 * KSTEPS);
+      dp = Mma<T>::run(bit_cast<V8>(fa[x]), bit_cast<V8>(fb[x]), dp);
+      if (x > KSTEPS) p_slice(x - KSTEPS - 1);
+      fence_order();
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) dv4[q] = lds_ld<f32x4>(st, 4 * kTileRows + 32 * q);
+    // dV^T += dO^T P, dK^T += Q^T dS: M = d, N = keys, k-step s2 covers rows
+    // 16s2 + 8(e/4) + 4lh + e%4 -- elements 8s2 .. 8s2+7 of the accumulator.
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      rt(g + VA);
+      dv[g >> 1] = Mma<T>::run(tr(g), pb[g & 1], dv[g >> 1]);
+      if (g == 0) p_slice(KSTEPS - 1);
+      else ds_slice(g - 1);
+      fence_order();
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (g + VA < NG) rt(NG + g + VA);
+      dk[g >> 1] = Mma<T>::run(tr(NG + g), db[g & 1], dk[g >> 1]);
+      if (g == 0) ds_slice(NG - 1);
+      fence_order();
+    }
   };
 
-  for (int n = 0; n < n_steps; ++n) {
-    const int s = n & (kBufs - 1);
-    const bool has = n < my_tiles;  // group 1 has no tile on the last step of an odd count
-    // Wait for this group's tile of step n (and on the first step the K / V
-    // blocks): vector memory completes in issue order, and in the steady
-    // state issued after this tile's loads are the next kBufs-2 tiles' loads.
-    if (n >= kBufs - 1 && n + kBufs - 2 < my_tiles)
-      vm_wait<(kBufs - 2) * LPW>();
-    else
+  // (one loop per kind of block, no branch around a step: a merge of
+  // accumulators inside the loop costs copies of all of them)
+  auto walk = [&](auto masked_c) {
+    for (int n = 0; n < my_tiles; ++n) {
+      const int s = n & (kBufs - 1);
+      // This group's tile of step n landed (and on the first step the K / V
+      // blocks); every wave is done with step n-1, whose buffers step n+1's
+      // tiles load into.
       vm_wait<0>();
-    // every wave is done with step n-1: its buffers (the ones step n+kBufs-1
-    // loads into) are free
-    sync_lds();
-    if (n + kBufs - 1 < my_tiles) issue_tile(tile_at(2 * (n + kBufs - 1) + rg), (n + kBufs - 1) & (kBufs - 1));
-    const unsigned char* qt = tiles + 2 * (rg * kBufs + s) * TILE_B;
-    const unsigned char* dot = qt + TILE_B;
-
-    if (has) {
-      // S = Q K^T, dP = dO V^T: M = rows, N = keys; lane (key ln, lh) holds
-      // rows 8(i/4) + 4lh + i%4 of its key.
-      f32x16 sc, dp;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sc[i] = dp[i] = 0.f;
-#pragma unroll
-      for (int kk = 0; kk < KSTEPS; ++kk) {
-        const int ro = r_off(kk);
-        const i16x8 qa = *reinterpret_cast<const i16x8*>(qt + ro);
-        const i16x8 kf = *reinterpret_cast<const i16x8*>(kmine + ro);
-        const i16x8 da = *reinterpret_cast<const i16x8*>(dot + ro);
-        const i16x8 vf = *reinterpret_cast<const i16x8*>(vmine + ro);
-        sc = Mma<T>::run(bit_cast<V8>(qa), bit_cast<V8>(kf), sc);
-        dp = Mma<T>::run(bit_cast<V8>(da), bit_cast<V8>(vf), dp);
-      }
-      // P and dS from the row statistics of the lane's 16 rows (one group of
-      // 4 rows at a time) and its key's mask word.
-      uint32_t w = key_ok ? 0xffffffffu : 0u;
-      if (tree_blk) w &= visw[(rg * kBufs + s) * kBlockKeys + 32 * kg + ln];
-      V8 pb[2], db[2];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float4* rp = reinterpret_cast<const float4*>(rs + (rg * kBufs + s) * kTileRows + 8 * q + 4 * lh);
-        const float4 st0 = rp[0], st1 = rp[1];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int i = 4 * q + e, m = 8 * q + 4 * lh + e;
-          const float4 pr = (e < 2) ? st0 : st1;
-          const float lse2 = (e & 1) ? pr.z : pr.x;
-          const float dvr = (e & 1) ? pr.w : pr.y;
-          const float p = ((w >> m) & 1u) ? __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], sl2, -lse2)) : 0.f;
-          pb[i >> 3][i & 7] = (T)p;
-          db[i >> 3][i & 7] = (T)(p * (dp[i] - dvr));
-        }
-      }
-      // dV^T += dO^T P, dK^T += Q^T dS: M = d, N = keys, k-step s2 covers rows
-      // 16s2 + 8(e/4) + 4lh + e%4 -- elements 8s2 .. 8s2+7 of the accumulator.
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          const i16x8 doT = tr_pair(dot + 16 * s2 * ROWB, dt);
-          const i16x8 qT = tr_pair(qt + 16 * s2 * ROWB, dt);
-          dv[dt] = Mma<T>::run(bit_cast<V8>(doT), pb[s2], dv[dt]);
-          dk[dt] = Mma<T>::run(bit_cast<V8>(qT), db[s2], dk[dt]);
-        }
+      sync_lds();
+      if (n + 1 < my_tiles) issue_tile(2 * (n + 1) + rg, s ^ 1);
+      tile_step(masked_c, s);
     }
+  };
+  if (all_keys) walk(std::false_type{});
+  else walk(std::true_type{});
+  if (my_tiles < n_steps) {  // group 1 has no tile on the last step of an odd count
+    vm_wait<0>();            // (a single tile: its share of the K / V blocks)
+    sync_lds();
   }
 
   // Row group 1 hands dK^T / dV^T to row group 0 through LDS (the K / V
@@ -405,8 +469,8 @@ constexpr int kRing = 4;     // LDS ring stages of 32-key units
 constexpr int kMaxDqSplits = 16;
 
 template <int D> constexpr size_t dq_lds_bytes() {
-  // kRing x (K unit, V unit, mask words of the chunk's 4 row tiles x 32 keys) | dummy load targets
-  return (size_t)kRing * (2 * 32 * D * 2 + 4 * 32 * 4) + 64;
+  // kRing x (K unit, V unit, mask words of the chunk's 4 row tiles x 32 keys, padded to 256 bytes)
+  return (size_t)kRing * (2 * 32 * D * 2 + 4 * 32 * 4);
 }
 
 // Wait until at most k units (LPU loads each) of this wave are in flight.
@@ -432,6 +496,15 @@ template <int LPU, int K> __device__ inline void wait_units(int k) {
 //   holds keys in; K^T from ds_read_b64_tr_b16 in the same order).
 // The workgroup's dQ^T adds to the fp32 accumulator once at the end
 // (atomics: several splits of one chunk add to the same rows).
+//
+// What bounds it: VALU issue and latency (40 % MFMA busy, 9.5 VALU per MFMA
+// at the 1024-token tree behind 16k keys when every unit built and tested a
+// visibility bit per score and the softmax sat between the MFMA groups).  A
+// unit runs S^T; dP^T with the exponentials between its MFMAs; dQ^T's first
+// half with the second half's dS between; whole prefix units compile
+// without the visibility tests and load at a scalar base plus fixed lane
+// offsets: 1.04 M -> 0.78 M cycles at that shape, 227 -> 88 VALU instructions
+// per 24 MFMAs.
 template <typename T, int D>
 __global__ __launch_bounds__(kQWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dq_main_kernel(const BwdArgs a) {
@@ -445,13 +518,11 @@ void bwd_dq_main_kernel(const BwdArgs a) {
   constexpr int VISB = 4 * 32 * 4;         // mask words of the chunk's 4 row tiles for the unit's 32 keys
   constexpr int SB = 2 * HALF + VISB;      // ring stage
   constexpr int LPH = HALF / 1024;         // 1 KB loads per half
-  constexpr int UPW = 2 * LPH / kQWaves;   // K + V loads per wave per unit
-  constexpr int LPU = UPW + 1;             // + the mask words (wave 0, tree units) or a dummy load
-  static_assert(UPW >= 1 && UPW * kQWaves == 2 * LPH, "load split");
+  constexpr int UPW = 2 * LPH / kQWaves;   // K + V loads per wave per unit (wave 0 of a tree unit: one more)
+  static_assert(UPW >= 1 && UPW * kQWaves == 2 * LPH && SB % 256 == 0, "load split, aligned stages");
 
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  extern __shared__ __attribute__((aligned(256))) unsigned char smem[];
   unsigned char* ring = smem;
-  unsigned char* dummy = ring + kRing * SB;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -501,9 +572,9 @@ void bwd_dq_main_kernel(const BwdArgs a) {
       df[kk] = *reinterpret_cast<const i16x8*>(dp + 16 * kk);
     }
     if (active) {
-      const float2 st = a.rowstat[(int64_t)bk * TGP + r];  // padding rows: (+inf, 0)
-      lse2 = st.x;
-      dvr = st.y;
+      const float* st = a.rowstat + ((int64_t)bk * a.n_tiles + tile) * (2 * kTileRows) + ln;
+      lse2 = st[0];  // padding rows: +inf, 0
+      dvr = st[kTileRows];
     }
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) asm volatile("" : : "v"(qf[kk]), "v"(df[kk]));
@@ -511,19 +582,33 @@ void bwd_dq_main_kernel(const BwdArgs a) {
   }
 
   auto key0_of = [&](int u) { return u < a.n_pu ? 32 * u : P + 32 * (u - a.n_pu); };
-  // HBM -> LDS: this wave's share of unit u into stage st.
+  // HBM -> LDS: this wave's share of unit u into stage st (waves 0, 1 move
+  // K, 2, 3 V).
+  const bool is_v = wave >= kQWaves / 2;
+  const T* ubase = is_v ? vbase : kbase;
+  const int64_t ustride = is_v ? a.svn : a.skn;
+  const int urow0 = (wave % (kQWaves / 2)) * UPW * RPL;
+  uint32_t uoff[UPW];  // key_fast: lane byte offsets from the unit's first key
+#pragma unroll
+  for (int i = 0; i < UPW; ++i) {
+    const int row = urow0 + i * RPL + lane / CPR;
+    uoff[i] = (uint32_t)(((int64_t)row * ustride + (((lane % CPR) ^ swz<D>(row)) << 3)) * 2);
+  }
   auto issue = [&](int st, int u) {
     unsigned char* sb = ring + st * SB;
     const int key0 = key0_of(u);
+    const uint32_t dst = lds_addr(sb + (is_v ? HALF : 0) + (wave % (kQWaves / 2)) * UPW * 1024);
+    if (a.key_fast && key0 + 32 <= a.kv_len) {
+      const T* src = ubase + (int64_t)key0 * ustride;
 #pragma unroll
-    for (int i = 0; i < UPW; ++i) {
-      const int v = wave * UPW + i;  // 0 .. 2*LPH-1: K loads, then V loads
-      const bool is_v = v >= LPH;
-      const int vl = is_v ? v - LPH : v;
-      const int row = vl * RPL + lane / CPR, pos = lane % CPR;
-      const int key = min(key0 + row, a.kv_len - 1);
-      const T* src = (is_v ? vbase + (int64_t)key * a.svn : kbase + (int64_t)key * a.skn) + ((pos ^ swz<D>(row)) << 3);
-      dma16(src, lds_addr(sb + (is_v ? HALF : 0) + vl * 1024));
+      for (int i = 0; i < UPW; ++i) dma16_s(src, uoff[i], dst + i * 1024);
+    } else {
+#pragma unroll
+      for (int i = 0; i < UPW; ++i) {
+        const int row = urow0 + i * RPL + lane / CPR;
+        const int key = min(key0 + row, a.kv_len - 1);
+        dma16(ubase + (int64_t)key * ustride + (((lane % CPR) ^ swz<D>(row)) << 3), dst + i * 1024);
+      }
     }
     if (wave == 0 && u >= a.n_pu) {
       // words [tile][tree key]: 4 tiles x 32 keys x 4 B, 8 lanes per tile
@@ -531,21 +616,18 @@ void bwd_dq_main_kernel(const BwdArgs a) {
         const int jt = min(chunk * kQWaves + (lane >> 3), a.n_tiles - 1);
         dma16(visbase + (int64_t)jt * a.n_tkeys + 32 * (u - a.n_pu) + 4 * (lane & 7), lds_addr(sb + 2 * HALF));
       }
-    } else if (lane == 0) {
-      dma16(a.rowstat, lds_addr(dummy + 16 * wave));
     }
   };
 
-  // LDS offsets: row reads of K / V (lane (key ln, lh), chunk 2kk + lh) and
-  // transposed reads of K (rows 8jj + 4(x>>1) + (i>>2), d = dt*32 + 16(x&1) +
-  // 4(i&3)); the tiles use the same swizzle as the dK / dV kernel.
+  // LDS offsets: row reads of K / V (lane (key ln, lh), chunk 2kk + lh) at
+  // r_off0 ^ (kk << 5), transposed reads of K (rows 8jj + 4(x>>1) + (i>>2), d
+  // = dt*32 + 16(x&1) + 4(i&3)) at (t_off0 ^ (dt << 6) ^ (jj << 5)) + 8jj
+  // rows; the tiles use the same swizzle as the dK / dV kernel.
   const int vx = lane >> 4, vi = lane & 15;
-  auto r_off = [&](int kk) { return ln * ROWB + (((2 * kk + lh) ^ swz<D>(ln)) << 4); };
-  auto t_off = [&](int dt, int jj) {
-    const int rr = 8 * jj + 4 * (vx >> 1) + (vi >> 2);
-    const int d = dt * 32 + 16 * (vx & 1) + 4 * (vi & 3);
-    return rr * ROWB + (((d >> 3) ^ swz<D>(rr)) << 4) + ((d & 7) << 1);
-  };
+  const int trow = 4 * (vx >> 1) + (vi >> 2);
+  const uint32_t r_off0 = (uint32_t)(ln * ROWB + ((lh ^ swz<D>(ln)) << 4));
+  const uint32_t t_off0 =
+      (uint32_t)(trow * ROWB + (((2 * (vx & 1) + ((vi & 3) >> 1)) ^ swz<D>(trow)) << 4) + ((vi & 1) << 3));
 
   f32x16 acc[DT];
 #pragma unroll
@@ -553,67 +635,116 @@ void bwd_dq_main_kernel(const BwdArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
 
-  for (int j = 0; j < kRing - 1 && j < mine; ++j) issue(j, u_lo + j);
-  for (int j = 0; j < mine; ++j) {
-    // unit j landed for every wave (later units in flight: up to kRing-2);
-    // every wave is done with unit j-1, whose stage unit j+kRing-1 reuses
-    wait_units<LPU, kRing - 2>(min(mine - 1 - j, kRing - 2));
-    sync_lds();
-    if (j + kRing - 1 < mine) issue((j + kRing - 1) % kRing, u_lo + j + kRing - 1);
-    if (!active) continue;
-    const unsigned char* sb = ring + (j % kRing) * SB;
-    const int u = u_lo + j;
-    const bool tree_u = u >= a.n_pu;
+  // One unit from the stage at LDS address sb.  masked_c: tree units and the
+  // prefix's partial last unit (vis16: the lane's 16 keys).
+  auto unit_step = [&](auto masked_c, uint32_t sb, uint32_t vis16) {
+    constexpr bool MASKED = decltype(masked_c)::value;
+    constexpr int RA = 4;            // row-operand reads ahead of their MFMA
+    constexpr int EP = 16 / KSTEPS;  // elements of P between two MFMAs
+    // (read offsets formed anew each unit, as in the dK / dV kernel)
+    uint32_t r0 = sb + r_off0, t0 = sb + t_off0;
+    asm volatile("" : "+v"(r0), "+v"(t0));
+    // operand x: K's k-steps (S^T), then V's (dP^T)
+    i16x8 f[2 * KSTEPS];
+    auto rd = [&](int x) {
+      f[x] = lds_ld<i16x8>(r0 ^ (uint32_t)((x % KSTEPS) << 5), x < KSTEPS ? 0 : HALF);
+    };
+    // transposed K pair x = s2 * DT + dt
+    i16x4 tl[2 * DT], th[2 * DT];
+    auto rt = [&](int x) {
+      const uint32_t c = t0 ^ (uint32_t)((x % DT) << 6);
+      tl[x] = lds_tr(c, 16 * (x / DT) * ROWB);
+      th[x] = lds_tr(c ^ 32u, (16 * (x / DT) + 8) * ROWB);
+    };
     // S^T = K Q^T, dP^T = V dO^T: M = keys, N = rows; lane (row ln, lh)
     // holds keys 8(i/4) + 4lh + i%4.
     f32x16 sc, dp;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) sc[i] = dp[i] = 0.f;
-#pragma unroll
-    for (int kk = 0; kk < KSTEPS; ++kk) {
-      const int ro = r_off(kk);
-      const i16x8 kf = *reinterpret_cast<const i16x8*>(sb + ro);
-      const i16x8 vf = *reinterpret_cast<const i16x8*>(sb + HALF + ro);
-      sc = Mma<T>::run(bit_cast<V8>(kf), bit_cast<V8>(qf[kk]), sc);
-      dp = Mma<T>::run(bit_cast<V8>(vf), bit_cast<V8>(df[kk]), dp);
-    }
-    // visibility of the lane's 16 keys from its row: prefix keys below P;
-    // tree keys: bit ln of each key's word for this wave's tile
-    uint32_t vis16 = 0;
-    if (tree_u) {
-      const uint32_t* wv = reinterpret_cast<const uint32_t*>(sb + 2 * HALF) + wave * 32;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint4 w4 = *reinterpret_cast<const uint4*>(wv + 8 * q + 4 * lh);
-        vis16 |= ((w4.x >> ln) & 1u) << (4 * q + 0);
-        vis16 |= ((w4.y >> ln) & 1u) << (4 * q + 1);
-        vis16 |= ((w4.z >> ln) & 1u) << (4 * q + 2);
-        vis16 |= ((w4.w >> ln) & 1u) << (4 * q + 3);
-      }
-    } else {
-      const int key0 = 32 * u;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) vis16 |= (uint32_t)(key0 + 8 * (i >> 2) + 4 * lh + (i & 3) < P) << i;
-    }
     V8 db[2];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float p = ((vis16 >> i) & 1u) ? __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], sl2, -lse2)) : 0.f;
-      db[i >> 3][i & 7] = (T)(p * (dp[i] - dvr));
+    for (int i = 0; i < 16; ++i) sc[i] = dp[i] = 0.f;
+    auto p_slice = [&](int y) {
+#pragma unroll
+      for (int i = EP * y; i < EP * (y + 1); ++i) {
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], sl2, -lse2));
+        sc[i] = MASKED && !((vis16 >> i) & 1u) ? 0.f : p;
+      }
+    };
+    auto ds = [&](int i) { db[i >> 3][i & 7] = (T)(sc[i] * (dp[i] - dvr)); };
+#pragma unroll
+    for (int x = 0; x < RA; ++x) rd(x);
+    fence_order();
+#pragma unroll
+    for (int x = 0; x < KSTEPS; ++x) {
+      rd(x + RA);
+      sc = Mma<T>::run(bit_cast<V8>(f[x]), bit_cast<V8>(qf[x]), sc);
+      fence_order();
     }
+#pragma unroll
+    for (int x = KSTEPS; x < 2 * KSTEPS; ++x) {
+      if (x + RA < 2 * KSTEPS) rd(x + RA);
+      else if (x + RA - 2 * KSTEPS < 2 * DT) rt(x + RA - 2 * KSTEPS);
+      dp = Mma<T>::run(bit_cast<V8>(f[x]), bit_cast<V8>(df[x - KSTEPS]), dp);
+      if (x > KSTEPS) p_slice(x - KSTEPS - 1);
+      fence_order();
+    }
+    p_slice(KSTEPS - 1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ds(i);
     // dQ^T += K^T dS^T: M = d, N = rows, k-step s2 covers keys 16s2 + 8(e/4)
     // + 4lh + e%4 -- elements 8s2 .. 8s2+7 of the accumulator.
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+    for (int x = 0; x < 2 * DT; ++x) {
+      if (x + RA < 2 * DT) rt(x + RA);
+      const i16x8 kT = __builtin_shufflevector(tl[x], th[x], 0, 1, 2, 3, 4, 5, 6, 7);
+      acc[x % DT] = Mma<T>::run(bit_cast<V8>(kT), db[x / DT], acc[x % DT]);
+      if (x < DT) {
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (TSFA_LDS i16x4*)(sb + 16 * s2 * ROWB + t_off(dt, 0)));
-        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (TSFA_LDS i16x4*)(sb + 16 * s2 * ROWB + t_off(dt, 1)));
-        const i16x8 kT = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        acc[dt] = Mma<T>::run(bit_cast<V8>(kT), db[s2], acc[dt]);
+        for (int i = 8 + 8 / DT * x; i < 8 + 8 / DT * (x + 1); ++i) ds(i);
       }
+      fence_order();
+    }
+  };
+
+  auto step = [&](int j) {
+    // unit j landed for every wave (later units in flight: up to kRing-2, at
+    // least UPW loads each); every wave is done with unit j-1, whose stage
+    // unit j+kRing-1 reuses
+    wait_units<UPW, kRing - 2>(min(mine - 1 - j, kRing - 2));
+    sync_lds();
+    if (j + kRing - 1 < mine) issue((j + kRing - 1) % kRing, u_lo + j + kRing - 1);
+    return lds_addr(ring + (j % kRing) * SB);
+  };
+  for (int j = 0; j < kRing - 1 && j < mine; ++j) issue(j, u_lo + j);
+  // whole prefix units, then the masked ones (a loop each: a merge of
+  // accumulators inside a loop costs copies of all of them)
+  const int n_full = min(max(P / 32 - u_lo, 0), mine);
+  if (active) {
+    for (int j = 0; j < n_full; ++j) unit_step(std::false_type{}, step(j), 0u);
+    for (int j = n_full; j < mine; ++j) {
+      const uint32_t sb = step(j);
+      const int u = u_lo + j;
+      // visibility of the lane's 16 keys from its row: prefix keys below P;
+      // tree keys: bit ln of each key's word for this wave's tile
+      uint32_t vis16 = 0;
+      if (u >= a.n_pu) {
+        const uint32_t wv = sb + 2 * HALF + wave * 128 + 16 * lh;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const u32x4 w4 = lds_ld<u32x4>(wv, 32 * q);
+          vis16 |= ((w4[0] >> ln) & 1u) << (4 * q + 0);
+          vis16 |= ((w4[1] >> ln) & 1u) << (4 * q + 1);
+          vis16 |= ((w4[2] >> ln) & 1u) << (4 * q + 2);
+          vis16 |= ((w4[3] >> ln) & 1u) << (4 * q + 3);
+        }
+      } else {
+        const int key0 = 32 * u;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) vis16 |= (uint32_t)(key0 + 8 * (i >> 2) + 4 * lh + (i & 3) < P) << i;
+      }
+      unit_step(std::true_type{}, sb, vis16);
+    }
+  } else {
+    for (int j = 0; j < mine; ++j) step(j);
   }
   // lane (row ln, lh) holds d = dt*32 + 8(i/4) + 4lh + i%4.  One split per
   // chunk: the workgroup owns its rows' dQ and writes it in the input dtype.
@@ -651,7 +782,7 @@ struct PrepArgs {
   const void* o;
   const void* dout;
   const float* lse;  // [B, Hq, q_len]
-  float2* rowstat;   // [B*Hkv][n_tiles*32]
+  float* rowstat;    // [B*Hkv][n_tiles][2][32]: log2 LSE, then Dv
   float* dq_acc;     // [B*Hkv][D][TGP]
   int64_t sob, soh, som, sdob, sdoh, sdom;
   int batch, num_heads, num_kv_heads, group, q_len, n_tiles;
@@ -696,7 +827,9 @@ __device__ inline void bwd_prep(const PrepArgs& a, int blk) {
   for (int off = 8; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 16);
   if (live && part == 0) {
     const bool empty = !(lse > -INFINITY);  // no visible key (or a padding row)
-    a.rowstat[row] = empty ? make_float2(INFINITY, 0.f) : make_float2(lse * 1.4426950408889634f, acc);
+    float* st = a.rowstat + (row / kTileRows) * (2 * kTileRows) + row % kTileRows;
+    st[0] = empty ? INFINITY : lse * 1.4426950408889634f;
+    st[kTileRows] = empty ? 0.f : acc;
   }
 }
 
@@ -944,7 +1077,7 @@ extern "C" int tsfa_bwd(const void* q, const void* k, const void* v, const void*
     return TSFA_ERR_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(workspace) % 256 != 0) return TSFA_ERR_WORKSPACE;
   char* ws = static_cast<char*>(workspace);
-  float2* rowstat = reinterpret_cast<float2*>(ws);
+  float* rowstat = reinterpret_cast<float*>(ws);
   float* dq_acc = reinterpret_cast<float*>(ws + p.rowstat_bytes);
   uint32_t* vis = reinterpret_cast<uint32_t*>(ws + p.rowstat_bytes + p.dq_bytes);
   const int tree_key_limit =
@@ -1067,6 +1200,13 @@ extern "C" int tsfa_bwd(const void* q, const void* k, const void* v, const void*
   pa.zero_dq = ba.dq_direct ? 0 : 1;
   ba.group_magic = gqa_group_size > 1 ? (uint32_t)((((uint64_t)1) << 32) / (uint64_t)gqa_group_size + 1) : 0u;
   ba.items_per_xcd = (ba.n_items + 7) / 8;
+  // a tile's (unit's) lanes reach this far past its first token (key), in bytes
+  auto lane_reach = [&](int64_t sh, int64_t sm) {
+    return 2 * ((gqa_group_size - 1) * sh + (kTileRows / gqa_group_size - 1) * sm + head_dim);
+  };
+  ba.tile_fast = 32 % gqa_group_size == 0 && lane_reach(ba.sqh, ba.sqm) < INT32_MAX &&
+                 lane_reach(ba.sdoh, ba.sdom) < INT32_MAX;
+  ba.key_fast = 2 * (31 * std::max(ba.skn, ba.svn) + head_dim) < INT32_MAX;
 
   DqArgs da;
   da.dq_acc = dq_acc;
