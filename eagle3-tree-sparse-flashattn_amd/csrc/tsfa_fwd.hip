@@ -156,6 +156,10 @@ struct SplitArgs {
   // split kernel writes O itself (ws_o is O; split_kernel<..., FAST | 4>)
   // and no combine runs.  Host-side only.
   int direct_out;
+  // The tree as a device mask (nonzero byte: visible) instead of the CSR
+  // record (split_kernel<..., FAST | 16>; the record's fields unused).
+  const uint8_t* mask;
+  int64_t mask_seq_stride, mask_row_stride;
 };
 
 
@@ -480,6 +484,7 @@ void split_kernel(const SplitArgs a) {
   constexpr int FM = FAST & 3;              // unchecked ring steps: 0 off, 1 plain, 2 non-temporal loads
   constexpr bool DIRECT = (FAST & 4) != 0;  // one-slot plan: write O, no combine
   constexpr bool PTAB = PAGED && FM != 0 && (FAST & 8) != 0;  // paged: steady refills from the LDS page-id table
+  constexpr bool MASK = (FAST & 16) != 0;   // the tree read from the mask itself, no CSR record
   typedef typename Mma<T>::vec8 V8;
   constexpr int RG = kWaves / S;             // row groups (waves per stream)
   constexpr int ROWS = 32 * RG;              // rows per chunk
@@ -1184,17 +1189,44 @@ void split_kernel(const SplitArgs a) {
     const int tok_hi = (int)fdiv(row0 + rows_chunk - 1, a.fd_group);  // tokens tok_lo .. tok_hi
     const int ntok = tok_hi - tok_lo + 1;
     const int qb_lo = tok_lo / BM, qb_hi = tok_hi / BM, nqbc = qb_hi - qb_lo + 1;
+    const int n_tu = (a.tree_key_limit + kUnitKeys - 1) / kUnitKeys;
     const int32_t* rp = a.row_ptr + b * a.ms_row_ptr;
     const int32_t* ci = a.col_idx + b * a.ms_col_idx;
     const int8_t* bt = a.blk_type + b * a.ms_blk_type;
     const int32_t* pl = a.payload + b * a.ms_payload;
     const int32_t* of = a.offset + b * a.ms_offset;
-    int* st = reinterpret_cast<int*>(ring);  // [nqbc][ntb]: 0 ZERO, -1 FULL, 1+offset MIXED
+    // [nqbc][ntb]: 0 ZERO, -1 FULL, 1+offset MIXED (MASK: [ntb], nonzero where
+    // a row of the chunk's q-blocks sees a key of the block)
+    int* st = reinterpret_cast<int*>(ring);
+    const int n_st = MASK ? ntb : nqbc * ntb;
+    // MASK: the packed mask rows of the chunk's q-blocks, [row][unit], behind
+    // the flags (at most kMaskWindowBytes / 8 and a word per row; the first
+    // unit loop overwrites them)
+    const uint8_t* mrow = MASK ? a.mask + b * a.mask_seq_stride : nullptr;
+    uint32_t* mw = reinterpret_cast<uint32_t*>(st + (MASK ? ntb : 0));
+    const int w_lo = qb_lo * BM, w_rows = min((qb_hi + 1) * BM, a.q_len) - w_lo;
     int* rps = misc + 8;                     // row_ptr[qb_lo .. qb_hi+1]
     // Block states of the chunk's q-blocks in two parallel round trips: the
     // row_ptr window, then every CSR entry of those rows at once.
+    // MASK: the q-blocks' rows packed straight from the mask, one round trip
+    // and no builder launch before this kernel (the 8B decode shape's verify
+    // call 17.8 -> 14.9 us); a block with a visible pair marks the units it
+    // overlaps, so the visited units are the CSR record's.
     auto build_state = [&]() {
-      for (int i = tid; i < nqbc * ntb; i += kWaves * 64) st[i] = 0;
+      for (int i = tid; i < n_st; i += kWaves * 64) st[i] = 0;
+      if constexpr (MASK) {
+        sync_lds();
+        for (int i = tid; i < w_rows * n_tu; i += kWaves * 64) {
+          const int row = i / n_tu, u = i - row * n_tu;
+          const uint32_t w = mask_word(mrow + (w_lo + row) * a.mask_row_stride, u * kUnitKeys, a.tree_key_limit);
+          mw[i] = w;
+          // BN is a multiple of 16: each 16-key half lies in one block
+          if (w & 0xffffu) st[u * kUnitKeys / BN] = 1;
+          if (w >> 16) st[(u * kUnitKeys + 16) / BN] = 1;
+        }
+        sync_lds();
+        return;
+      }
       if (tid <= nqbc) rps[tid] = rp[qb_lo + tid];
       sync_lds();
       const int e_begin = rps[0], e_end = rps[nqbc];
@@ -1209,10 +1241,9 @@ void split_kernel(const SplitArgs a) {
     build_state();
     TSFA_STAMP(44);
     // Tree units holding a key some row of the chunk can see, compacted.
-    const int n_tu = (a.tree_key_limit + kUnitKeys - 1) / kUnitKeys;
     for (int i = tid; i < n_tu; i += kWaves * 64) vis[i] = 0;
     sync_lds();
-    for (int i = tid; i < nqbc * ntb; i += kWaves * 64) {
+    for (int i = tid; i < n_st; i += kWaves * 64) {
       if (st[i] != 0) {
         const int tb = i % ntb;
         const int c_first = tb * BN, c_last = min(tb * BN + BN, a.tree_key_limit) - 1;
@@ -1238,9 +1269,15 @@ void split_kernel(const SplitArgs a) {
     for (int vb0 = 0; vb0 < n_vis; vb0 += a.vt_max) {
       const int nb = min(a.vt_max, n_vis - vb0);
       if (vb0 > 0) build_state();
+      if constexpr (MASK) {
+        for (int it = tid; it < ntok * nb; it += kWaves * 64) {
+          const int tt = it / nb, j = it - tt * nb;
+          masks[tt * a.vt_max + j] = mw[(tok_lo + tt - w_lo) * n_tu + vis[vb0 + j]];
+        }
+      }
       // Per-token visibility word of each unit of the batch, from two 16-key
       // groups (BN is a multiple of 16, so a group never straddles blocks).
-      for (int it = tid; it < ntok * nb * 2; it += kWaves * 64) {
+      for (int it = tid; !MASK && it < ntok * nb * 2; it += kWaves * 64) {
         const int q2 = it & 1, jt = it >> 1;
         const int j = jt % nb, tt = jt / nb;
         const int t = tok_lo + tt, qb = t / BM, tl = t - qb * BM;
@@ -1547,6 +1584,16 @@ template <int D> inline int fast_ring(const SplitArgs& sa, const Plan& p, const 
   return p.streams == 2 ? 2 : 0;
 }
 
+// Mask bytes of a chunk's q-blocks that split_kernel<..., FAST | 16> packs:
+// each (batch, kv head, chunk) reads its own, so past this the builder, which
+// packs a mask once, is the cheaper way (and the packed words, an eighth of
+// it and a word per row, fit the LDS ring).  Whole calls behind a 2048-key
+// prefix, builder / mask: 294 KB (1024 tokens, one head per kv head) 78.0 /
+// 78.1 us, 393 KB 75.7 / 78.4 (one head per kv head) and 166.5 / 157.7 (2048
+// tokens, four), 576 KB (1500 tokens) 89.4 / 103.3; 196 KB (1024 tokens, four
+// heads, 16384 keys) 290 / 277.
+constexpr int64_t kMaskWindowBytes = 256 * 1024;
+
 // The kernels of one call, for the switches of one configuration snapshot
 // (cfg, read once by the caller).
 template <typename T, int D, bool PAGED>
@@ -1603,14 +1650,23 @@ int launch_all(const SplitArgs& sa_in, const CombineArgs& ca, const Plan& p, con
                                                  : launch_split<T, D, 1, true, false, 1>(sa, p, stream))
                                          : launch_split<T, D, 1, true, false>(sa, p, stream));
     else
-      st = p.streams == 2 ? (fm == 6   ? launch_split<T, D, 2, false, false, 6>(sa, p, stream)
-                             : fm == 5 ? launch_split<T, D, 2, false, false, 5>(sa, p, stream)
-                             : fm == 2 ? launch_split<T, D, 2, false, false, 2>(sa, p, stream)
-                             : fm == 1 ? launch_split<T, D, 2, false, false, 1>(sa, p, stream)
-                                       : launch_split<T, D, 2, false, false>(sa, p, stream))
-                          : (fm == 5   ? launch_split<T, D, 1, false, false, 5>(sa, p, stream)
-                             : fm == 1 ? launch_split<T, D, 1, false, false, 1>(sa, p, stream)
-                                       : launch_split<T, D, 1, false, false>(sa, p, stream));
+    {
+      auto go = [&](auto s_c, auto f_c) {
+        constexpr int S = decltype(s_c)::value, F = decltype(f_c)::value;
+        return sa.mask != nullptr ? launch_split<T, D, S, false, false, F | 16>(sa, p, stream)
+                                  : launch_split<T, D, S, false, false, F>(sa, p, stream);
+      };
+      auto with = [&](auto s_c) {
+        if constexpr (decltype(s_c)::value == 2) {
+          if (fm == 6) return go(s_c, std::integral_constant<int, 6>{});
+          if (fm == 2) return go(s_c, std::integral_constant<int, 2>{});
+        }
+        if (fm == 5) return go(s_c, std::integral_constant<int, 5>{});
+        if (fm == 1) return go(s_c, std::integral_constant<int, 1>{});
+        return launch_split<T, D, decltype(s_c)::value, false, false>(sa, p, stream);
+      };
+      st = p.streams == 2 ? with(std::integral_constant<int, 2>{}) : with(std::integral_constant<int, 1>{});
+    }
     if (st != TSFA_OK) return st;
   }
   // no combine when the split kernel wrote O
@@ -2264,6 +2320,37 @@ struct KvSource {
   bool paged() const { return cache != nullptr; }
 };
 
+// The tree of a call: its metadata arrays, or (mask set) a device mask and
+// the workspace sections that its metadata goes to where a kernel needs it.
+struct TreeSource {
+  const int32_t* row_ptr = nullptr;
+  const int32_t* col_idx = nullptr;
+  const int8_t* blk_type = nullptr;
+  const int32_t* payload = nullptr;
+  const int32_t* offset = nullptr;
+  const int64_t* seq_stride = nullptr;  // [5]
+  const uint8_t* mask = nullptr;
+  int64_t mask_seq_stride = 0, mask_row_stride = 0;
+  int n_masks = 0;
+  void* counts = nullptr;
+  void* build_ws = nullptr;
+  size_t build_ws_bytes = 0;
+
+  TreeSource() = default;
+  TreeSource(const int32_t* rp, const int32_t* ci, const int8_t* bt, const int32_t* pl, const int32_t* of,
+             const int64_t* ss)
+      : row_ptr(rp), col_idx(ci), blk_type(bt), payload(pl), offset(of), seq_stride(ss) {}
+
+  // The metadata arrays written from the mask, in stream order.
+  int build(int q_len, int block_m, int block_n, tsfa_stream_t stream) const {
+    return tsfa_meta_build(mask, mask_seq_stride, mask_row_stride, n_masks, q_len, block_m, block_n,
+                           const_cast<int32_t*>(row_ptr), const_cast<int32_t*>(col_idx),
+                           const_cast<int8_t*>(blk_type), const_cast<int32_t*>(payload),
+                           const_cast<int32_t*>(offset), static_cast<int32_t*>(counts), build_ws, build_ws_bytes,
+                           stream);
+  }
+};
+
 // The generic kernel's call (head_dim 256, fp32): contiguous K/V only.
 int gen_impl(const void* q, const KvSource& kv, void* o, float* lse, const int32_t* row_ptr, const int32_t* col_idx,
              const int8_t* blk_type, const int32_t* payload, const int32_t* offset, const int64_t* meta_seq_stride,
@@ -2349,9 +2436,8 @@ int gen_impl(const void* q, const KvSource& kv, void* o, float* lse, const int32
                                   : launch_gen<_Float16, 256>(ga, ca, p, stream);
 }
 
-int fwd_impl(const void* q, const KvSource& kv, void* o, float* lse, const int32_t* row_ptr, const int32_t* col_idx,
-             const int8_t* blk_type, const int32_t* mixed_mask_payload, const int32_t* mixed_mask_offset,
-             const int64_t* meta_seq_stride, const int64_t* q_strides, const int64_t* o_strides, float sm_scale,
+int fwd_impl(const void* q, const KvSource& kv, void* o, float* lse, const TreeSource& tree,
+             const int64_t* q_strides, const int64_t* o_strides, float sm_scale,
              int batch, int num_heads, int num_kv_heads, int q_len, int kv_len, int prefix_len, int n_q_blocks,
              int n_tree_blocks, int gqa_group_size, int block_m, int block_n, int head_dim, int dtype,
              void* workspace, size_t workspace_bytes, tsfa_stream_t stream_) {
@@ -2359,8 +2445,9 @@ int fwd_impl(const void* q, const KvSource& kv, void* o, float* lse, const int32
                                n_tree_blocks, gqa_group_size, block_m, block_n, head_dim, dtype);
   if (st != TSFA_OK) return st;
   if (batch == 0 || q_len == 0) return TSFA_OK;
+  const int64_t* meta_seq_stride = tree.seq_stride;
   if (q_strides == nullptr || o_strides == nullptr || meta_seq_stride == nullptr) return TSFA_ERR_INVALID_ARGUMENT;
-  if (q == nullptr || o == nullptr || row_ptr == nullptr) return TSFA_ERR_INVALID_ARGUMENT;
+  if (q == nullptr || o == nullptr || tree.row_ptr == nullptr) return TSFA_ERR_INVALID_ARGUMENT;
   if (kv.paged() && kv.kv_indices == nullptr) return TSFA_ERR_INVALID_ARGUMENT;
   if (kv.paged() && (kv.cache == nullptr || kv.cache_strides == nullptr)) return TSFA_ERR_INVALID_ARGUMENT;
   st = check_strides(q, q_strides, o, o_strides);
@@ -2371,11 +2458,14 @@ int fwd_impl(const void* q, const KvSource& kv, void* o, float* lse, const int32
   if (st != TSFA_OK) return st;
   for (int i = 0; i < 5; ++i)
     if (meta_seq_stride[i] < 0) return TSFA_ERR_INVALID_ARGUMENT;
-  if (gen_path(head_dim, dtype))
-    return gen_impl(q, kv, o, lse, row_ptr, col_idx, blk_type, mixed_mask_payload, mixed_mask_offset,
+  if (gen_path(head_dim, dtype)) {
+    if (tree.mask != nullptr) st = tree.build(q_len, block_m, block_n, stream_);
+    if (st != TSFA_OK) return st;
+    return gen_impl(q, kv, o, lse, tree.row_ptr, tree.col_idx, tree.blk_type, tree.payload, tree.offset,
                     meta_seq_stride, o_strides, sm_scale, batch, num_heads, num_kv_heads, q_len, kv_len, prefix_len,
                     gqa_group_size, block_m, block_n, head_dim, dtype, workspace, workspace_bytes,
                     reinterpret_cast<hipStream_t>(stream_), q_strides);
+  }
 
   // one snapshot of the TSFA_* switches for the whole call
   const Config cfg = config();
@@ -2388,11 +2478,11 @@ int fwd_impl(const void* q, const KvSource& kv, void* o, float* lse, const int32
 
   SplitArgs sa = {};
   sa.q = q;
-  sa.row_ptr = row_ptr;
-  sa.col_idx = col_idx;
-  sa.blk_type = blk_type;
-  sa.payload = mixed_mask_payload;
-  sa.offset = mixed_mask_offset;
+  sa.row_ptr = tree.row_ptr;
+  sa.col_idx = tree.col_idx;
+  sa.blk_type = tree.blk_type;
+  sa.payload = tree.payload;
+  sa.offset = tree.offset;
   sa.ms_row_ptr = meta_seq_stride[0];
   sa.ms_col_idx = meta_seq_stride[1];
   sa.ms_blk_type = meta_seq_stride[2];
@@ -2490,6 +2580,23 @@ int fwd_impl(const void* q, const KvSource& kv, void* o, float* lse, const int32
                        o_strides[0] == (int64_t)num_heads * q_len * head_dim;
   sa.direct_out = p.n_slots == 1 && lse == nullptr && o_dense && cfg.direct_out != 0 ? 1 : 0;
 
+  // A mask is read by the split kernel itself where an instance with the
+  // unchecked prefix steps runs and the chunks' windows are small; else its
+  // metadata is built first.
+  const bool bf = dtype == TSFA_DTYPE_BF16, d128 = head_dim == 128;
+  if (tree.mask != nullptr) {
+    const int64_t window = std::min<int64_t>(chunk_qblocks(p.rows_per_chunk, gqa_group_size, block_m) * block_m,
+                                             q_len) * q_len;
+    if (window <= kMaskWindowBytes && (d128 ? fast_ring<128>(sa, p, cfg) : fast_ring<64>(sa, p, cfg)) != 0) {
+      sa.mask = tree.mask;
+      sa.mask_seq_stride = tree.n_masks > 1 ? tree.mask_seq_stride : 0;
+      sa.mask_row_stride = tree.mask_row_stride;
+    } else {
+      st = tree.build(q_len, block_m, block_n, stream_);
+      if (st != TSFA_OK) return st;
+    }
+  }
+
   CombineArgs ca;
   ca.o = o;
   ca.lse = lse;
@@ -2507,7 +2614,6 @@ int fwd_impl(const void* q, const KvSource& kv, void* o, float* lse, const int32
   ca.ws_ml = sa.ws_ml;
 
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
-  const bool bf = dtype == TSFA_DTYPE_BF16, d128 = head_dim == 128;
   if (kv.paged()) {
     if (bf) return d128 ? launch_all<__bf16, 128, true>(sa, ca, p, cfg, stream) : launch_all<__bf16, 64, true>(sa, ca, p, cfg, stream);
     return d128 ? launch_all<_Float16, 128, true>(sa, ca, p, cfg, stream) : launch_all<_Float16, 64, true>(sa, ca, p, cfg, stream);
@@ -2530,17 +2636,18 @@ extern "C" int tsfa_fwd(const void* q, const void* k, const void* v, void* o, co
   kv.v = v;
   kv.k_strides = strides ? strides + 4 : nullptr;
   kv.v_strides = strides ? strides + 8 : nullptr;
-  return fwd_impl(q, kv, o, nullptr, row_ptr, col_idx, blk_type, mixed_mask_payload, mixed_mask_offset,
-                  meta_seq_stride, strides, strides ? strides + 12 : nullptr, sm_scale, batch, num_heads, num_kv_heads, q_len,
+  return fwd_impl(q, kv, o, nullptr, TreeSource(row_ptr, col_idx, blk_type, mixed_mask_payload, mixed_mask_offset,
+                  meta_seq_stride), strides, strides ? strides + 12 : nullptr, sm_scale, batch, num_heads, num_kv_heads, q_len,
                   kv_len, prefix_len, n_q_blocks, n_tree_blocks, gqa_group_size, block_m, block_n, head_dim, dtype,
                   workspace, workspace_bytes, stream_);
 }
 
 // ------------------------------------- metadata build + forward in one call
-// run_tree_sparse_kernel(q, k, v, tree_mask) as one C call: the device
-// metadata builder (tsfa_meta_build) writes the capacity-layout tree record
-// into the front of the workspace and the forward reads it there, in stream
-// order, with no host synchronisation.  Workspace layout (each section
+// run_tree_sparse_kernel(q, k, v, tree_mask) as one C call, with no host
+// synchronisation: the split kernel reads the mask itself where it can
+// (kMaskWindowBytes); else the device metadata builder (tsfa_meta_build)
+// writes the capacity-layout tree record into the front of the workspace and
+// the forward reads it there, in stream order.  Workspace layout (each section
 // 256-byte aligned): row_ptr, col_idx, blk_type, payload, offset, counts of
 // n_masks trees, the builder's scratch, the forward's split-KV partials.
 namespace {
@@ -2618,21 +2725,27 @@ extern "C" int tsfa_tree_attention(const void* q, const void* k, const void* v, 
   if (workspace == nullptr || workspace_bytes < L.total || reinterpret_cast<uintptr_t>(workspace) % 256 != 0)
     return TSFA_ERR_WORKSPACE;
   char* ws = static_cast<char*>(workspace);
-  int32_t* row_ptr = reinterpret_cast<int32_t*>(ws + L.off[0]);
-  int32_t* col_idx = reinterpret_cast<int32_t*>(ws + L.off[1]);
-  int8_t* blk_type = reinterpret_cast<int8_t*>(ws + L.off[2]);
-  int32_t* payload = reinterpret_cast<int32_t*>(ws + L.off[3]);
-  int32_t* offset = reinterpret_cast<int32_t*>(ws + L.off[4]);
-  int32_t* counts = reinterpret_cast<int32_t*>(ws + L.off[5]);
-  st = tsfa_meta_build(mask, mask_seq_stride, mask_row_stride, n_masks, q_len, block_m, block_n, row_ptr, col_idx,
-                       blk_type, payload, offset, counts, ws + L.off[6], L.off[7] - L.off[6], stream);
-  if (st != TSFA_OK) return st;
   // one tree for the batch: stride 0; one per sequence: the capacity layout
   const int64_t ms[5] = {n_masks > 1 ? (int64_t)L.nqb + 1 : 0, n_masks > 1 ? L.cap : 0, n_masks > 1 ? L.cap : 0,
                          n_masks > 1 ? L.cap * L.words : 0, n_masks > 1 ? L.cap : 0};
-  return tsfa_fwd(q, k, v, o, row_ptr, col_idx, blk_type, payload, offset, ms, strides, sm_scale, batch, num_heads,
-                  num_kv_heads, q_len, kv_len, prefix_len, L.nqb, L.ntb, num_heads / num_kv_heads, block_m, block_n,
-                  head_dim, dtype, ws + L.off[7], L.fwd_bytes, stream);
+  TreeSource tree(reinterpret_cast<int32_t*>(ws + L.off[0]), reinterpret_cast<int32_t*>(ws + L.off[1]),
+                  reinterpret_cast<int8_t*>(ws + L.off[2]), reinterpret_cast<int32_t*>(ws + L.off[3]),
+                  reinterpret_cast<int32_t*>(ws + L.off[4]), ms);
+  tree.mask = mask;
+  tree.mask_seq_stride = mask_seq_stride;
+  tree.mask_row_stride = mask_row_stride;
+  tree.n_masks = n_masks;
+  tree.counts = ws + L.off[5];
+  tree.build_ws = ws + L.off[6];
+  tree.build_ws_bytes = L.off[7] - L.off[6];
+  KvSource kv;
+  kv.k = k;
+  kv.v = v;
+  kv.k_strides = strides + 4;
+  kv.v_strides = strides + 8;
+  return fwd_impl(q, kv, o, nullptr, tree, strides, strides + 12, sm_scale, batch, num_heads, num_kv_heads, q_len,
+                  kv_len, prefix_len, L.nqb, L.ntb, num_heads / num_kv_heads, block_m, block_n, head_dim, dtype,
+                  ws + L.off[7], L.fwd_bytes, stream);
 }
 
 // ------------------------------------------------- allocation-free forward
@@ -2717,8 +2830,8 @@ extern "C" int tsfa_fwd_lse(const void* q, const void* k, const void* v, void* o
   kv.v = v;
   kv.k_strides = strides ? strides + 4 : nullptr;
   kv.v_strides = strides ? strides + 8 : nullptr;
-  return fwd_impl(q, kv, o, lse, row_ptr, col_idx, blk_type, mixed_mask_payload, mixed_mask_offset,
-                  meta_seq_stride, strides, strides ? strides + 12 : nullptr, sm_scale, batch, num_heads,
+  return fwd_impl(q, kv, o, lse, TreeSource(row_ptr, col_idx, blk_type, mixed_mask_payload, mixed_mask_offset,
+                  meta_seq_stride), strides, strides ? strides + 12 : nullptr, sm_scale, batch, num_heads,
                   num_kv_heads, q_len, kv_len, prefix_len, n_q_blocks, n_tree_blocks, gqa_group_size, block_m,
                   block_n, head_dim, dtype, workspace, workspace_bytes, stream_);
 }
@@ -2743,8 +2856,8 @@ extern "C" int tsfa_fwd_paged(const void* q, const void* kv_cache, const int32_t
   kv.pt_stride = page_table_stride;
   kv.n_pages = n_pages;
   kv.page_size = page_size;
-  return fwd_impl(q, kv, o, lse, row_ptr, col_idx, blk_type, mixed_mask_payload, mixed_mask_offset,
-                  meta_seq_stride, q_strides, o_strides, sm_scale, batch, num_heads, num_kv_heads, q_len, kv_len, prefix_len,
+  return fwd_impl(q, kv, o, lse, TreeSource(row_ptr, col_idx, blk_type, mixed_mask_payload, mixed_mask_offset,
+                  meta_seq_stride), q_strides, o_strides, sm_scale, batch, num_heads, num_kv_heads, q_len, kv_len, prefix_len,
                   n_q_blocks, n_tree_blocks, gqa_group_size, block_m, block_n, head_dim, dtype, workspace,
                   workspace_bytes, stream_);
 }

@@ -36,6 +36,39 @@ template <> struct Mma<_Float16> {
   }
 };
 
+// ------------------------------------------------------------- mask packing
+// Nonzero bytes of x (4 mask bytes, first byte lowest) as bits 0-3: the
+// high bit of each byte of (x & 0x7f7f7f7f) + 0x7f7f7f7f | x is set iff the
+// byte is nonzero; the multiply moves bits 7, 15, 23, 31 to 28..31 (its other
+// partial products land on distinct positions below 28, so no carry reaches
+// them).
+__device__ inline uint32_t nonzero_nibble(uint32_t x) {
+  const uint32_t t = ((((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u);
+  return (t * 0x00204081u) >> 28;
+}
+
+// 32 mask bytes from p (any alignment) as bits.
+__device__ inline uint32_t pack32(const uint8_t* p) {
+  uint32_t x[8];
+  __builtin_memcpy(x, p, 32);
+  uint32_t word = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) word |= nonzero_nibble(x[i]) << (4 * i);
+  return word;
+}
+
+// Columns [c0, c0 + 32) of one mask row as bits, columns from n on 0 (c0 < n):
+// two vector loads, those of the row's cut last word ending at column n; the
+// byte loads are for rows of fewer than 32 columns.
+__device__ inline uint32_t mask_word(const uint8_t* row, int c0, int n) {
+  const int valid = min(32, n - c0);
+  if (c0 + valid >= 32) return pack32(row + c0 + valid - 32) >> (32 - valid);
+  uint32_t word = 0;
+#pragma unroll
+  for (int i = 0; i < 32; ++i) word |= (uint32_t)(i < valid && row[c0 + min(i, valid - 1)] != 0) << i;
+  return word;
+}
+
 // ---------------------------------------------------------- host utilities
 int device_cu_count(int* out);            // cached per device
 int device_max_lds_per_block(int* out);   // cached per device

@@ -44,26 +44,6 @@ constexpr int kSmallWords = 8192;  // 32 KB of packed words in LDS
 constexpr int kTreeBlocks = 64;    // one wave's lanes
 constexpr int kPlaceGroups = 512;  // workgroups per sequence of the place kernel
 
-// Nonzero bytes of x (4 mask bytes, first byte lowest) as bits 0-3: the
-// high bit of each byte of (x & 0x7f7f7f7f) + 0x7f7f7f7f | x is set iff the
-// byte is nonzero; the multiply moves bits 7, 15, 23, 31 to 28..31 (its other
-// partial products land on distinct positions below 28, so no carry reaches
-// them).
-__device__ inline uint32_t nonzero_nibble(uint32_t x) {
-  const uint32_t t = ((((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u);
-  return (t * 0x00204081u) >> 28;
-}
-
-// 32 mask bytes from p (any alignment) as bits.
-__device__ inline uint32_t pack32(const uint8_t* p) {
-  uint32_t x[8];
-  __builtin_memcpy(x, p, 32);
-  uint32_t word = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) word |= nonzero_nibble(x[i]) << (4 * i);
-  return word;
-}
-
 // Bits [32*wi, 32*wi + 32) of block (qb, tb) of the sequence whose mask
 // starts at m0, zero-padded past the block's clipped h x w extent (:44-64).
 // (r0, c0): row and column of the word's first bit, flat = 32 * wi.

@@ -234,8 +234,9 @@ int tsfa_fwd_paged(const void* q, const void* kv_cache, const int32_t* kv_indptr
 /* run_tree_sparse_kernel(q, k, v, tree_mask) in one call
  * (eagle_tree_sparse_bridge.py:76-159: metadata from the tree mask, then the
  * forward with prefix_len = kv_len - q_len, eagle_tree_sparse_bridge.py:91-117):
- * tsfa_meta_build on the device mask into the front of `workspace`, then
- * tsfa_fwd reading that record, both on `stream`, no host synchronisation.
+ * tsfa_fwd's kernels reading the device mask themselves, or tsfa_meta_build on
+ * it into the front of `workspace` and tsfa_fwd reading that record (large
+ * trees), on `stream`, no host synchronisation.
  * mask      uint8 (nonzero = visible) device memory: n_masks trees of
  *           [q_len, q_len] rows mask_row_stride apart, trees mask_seq_stride
  *           apart; n_masks = 1 (one tree for the batch, as the reference) or

@@ -211,3 +211,31 @@ def test_one_call_path_refuses_kv_shorter_than_q():
     with pytest.raises(ValueError):
         bridge.run_tree_sparse_kernel(q.cuda(), k[:, :, :30].cuda(), v[:, :, :30].cuda(), mask.cuda(),
                                       block_m=16, block_n=32)
+
+
+# the split kernel's own mask read (tiles of 32 columns, cut and short rows,
+# q-blocks wider than a chunk, several word batches per chunk, one and two key
+# streams, one-slot plans, trees without a prefix) against the metadata route:
+# the same units in the same order, so the same bits
+@pytest.mark.parametrize("b,hq,hkv,t,p,d,bm,bn", [
+    (1, 4, 4, 1, 64, 64, 64, 64), (1, 4, 2, 7, 96, 128, 16, 16), (2, 8, 8, 31, 33, 64, 64, 48),
+    (3, 14, 2, 33, 1024, 64, 64, 64), (1, 32, 8, 61, 4095, 128, 16, 32), (16, 8, 2, 64, 2048, 128, 16, 64),
+    (1, 8, 1, 200, 500, 128, 128, 128), (2, 4, 1, 95, 0, 128, 32, 64), (1, 4, 2, 1100, 640, 64, 16, 64),
+    (1, 2, 2, 1200, 320, 128, 64, 64), (1, 8, 1, 515, 2048, 128, 1, 16)])
+def test_mask_read_in_the_kernel_matches_the_metadata_route(b, hq, hkv, t, p, d, bm, bn):
+    print(f"[bridge] mask read b={b} hq={hq} hkv={hkv} t={t} p={p} d={d} bm={bm} bn={bn}", flush=True)
+    rng = np.random.default_rng(t)
+    masks = np.stack([trees.ancestor_mask(trees.depth_limited_parents(t, 6, rng)) for _ in range(b)])
+    masks[0, t // 2] = False  # a row that sees no tree key
+    masks[-1, : min(t, 2 * bm), : min(t, bn)] = True
+    wide = torch.zeros((b, t, t + 3), dtype=torch.bool, device="cuda")
+    wide[:, :, 1:1 + t] = torch.from_numpy(masks).cuda()
+    mask = wide[:, :, 1:1 + t]  # unaligned rows
+    g = torch.Generator(device="cuda").manual_seed(t)
+    q, k, v = (torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)
+               for s in ((b, hq, t, d), (b, hkv, p + t, d), (b, hkv, p + t, d)))
+    for m in (mask, mask[0]):
+        got = bridge.run_tree_sparse_kernel(q, k, v, m, block_m=bm, block_n=bn)
+        meta = bridge.build_tree_metadata(m, p, bm, bn)
+        want = bridge.run_tree_sparse_kernel(q, k, v, None, block_m=bm, block_n=bn, metadata=meta)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))

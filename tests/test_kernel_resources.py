@@ -25,12 +25,15 @@ TARGET = "hipv4-amdgcn-amd-amdhsa--gfx950"
 
 # split_kernel<T, 128, S, PAGED, C32, FAST> -> most SGPR spills allowed.
 # FAST: 0 checked steps, 1/2 unchecked (plain / non-temporal loads), +4 the
-# one-slot kernel that writes O, +8 the paged page-id table.
+# one-slot kernel that writes O, +8 the paged page-id table, +16 the mask read.
 SPLIT_CEILINGS = {
     # contiguous: 8B decode (2, FAST 2), batched decode (2, 6), wide tree
     # (1, 1), 70B (1, 5), and the checked steps
     (2, False, False, 2): 19, (2, False, False, 1): 19, (2, False, False, 6): 17, (2, False, False, 5): 17,
     (2, False, False, 0): 42, (1, False, False, 1): 17, (1, False, False, 5): 17, (1, False, False, 0): 55,
+    # the same with the tree read from the mask (+16)
+    (2, False, False, 18): 8, (2, False, False, 17): 8, (2, False, False, 22): 7, (2, False, False, 21): 7,
+    (1, False, False, 17): 3, (1, False, False, 21): 3,
     # paged, 32-bit offsets (two streams) and 64-bit (two streams, one stream)
     (2, True, True, 9): 35, (2, True, True, 13): 36, (2, True, True, 1): 43, (2, True, True, 5): 39,
     (2, True, True, 0): 46, (2, True, False, 13): 34, (2, True, False, 1): 42, (2, True, False, 5): 38,
