@@ -1759,6 +1759,8 @@ struct GenArgs {
   void* out;       // direct: O [B, Hq, q_len, D] (strides sob, soh, som; d stride 1)
   int64_t sob, soh, som;
   int direct;      // one split and no LSE: the kernel writes O, no partials, no combine
+  const uint8_t* mask;  // the tree as a device mask (nonzero byte: visible) instead of the CSR record, or null
+  int64_t mask_seq_stride, mask_row_stride;
 };
 
 // 128-row chunks: 4 row groups of 32.  The 16-bit instances (head_dim 256)
@@ -1848,16 +1850,19 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
   const int32_t* pl = a.payload + b * a.ms[3];
   const int32_t* of = a.offset + b * a.ms[4];
   const int qb = t / a.block_m, tl = t - qb * a.block_m;
-  const int e_lo = rp[qb], e_hi = rp[qb + 1];
+  const uint8_t* mrow = a.mask != nullptr ? a.mask + b * a.mask_seq_stride + t * a.mask_row_stride : nullptr;
+  const int e_lo = mrow != nullptr ? 0 : rp[qb], e_hi = mrow != nullptr ? 0 : rp[qb + 1];
   // Visibility of keys k0 .. k0+31 for the lane's row: prefix keys, then the
-  // tree keys of the row's FULL and MIXED blocks (tree_sparse_flashattn.py:
+  // tree keys of the mask's row, or of the row's FULL and MIXED blocks (tree_sparse_flashattn.py:
   // 266-270, :307-318); keys past kv_len are not visible.
   auto vis_word = [&](int k0) {
     const int P = a.prefix_len, BN = a.block_n;
     const int np = min(max(P - k0, 0), 32);
     uint32_t w = np >= 32 ? 0xffffffffu : ((1u << np) - 1u);
     const int c_lo = max(k0, P) - P, c_hi = min(k0 + 32, a.kv_len) - P;  // tree columns of the unit
-    if (c_lo < c_hi) {
+    if (c_lo < c_hi && mrow != nullptr) {
+      w |= mask_word(mrow, c_lo, a.kv_len - P) << (c_lo + P - k0);
+    } else if (c_lo < c_hi) {
       for (int e = e_lo; e < e_hi; ++e) {
         const int cb = ci[e] * BN;
         const int lo = max(cb, c_lo), hi = min(cb + BN, c_hi);
@@ -2352,8 +2357,7 @@ struct TreeSource {
 };
 
 // The generic kernel's call (head_dim 256, fp32): contiguous K/V only.
-int gen_impl(const void* q, const KvSource& kv, void* o, float* lse, const int32_t* row_ptr, const int32_t* col_idx,
-             const int8_t* blk_type, const int32_t* payload, const int32_t* offset, const int64_t* meta_seq_stride,
+int gen_impl(const void* q, const KvSource& kv, void* o, float* lse, const TreeSource& tree,
              const int64_t* o_strides, float sm_scale, int batch, int num_heads, int num_kv_heads, int q_len,
              int kv_len, int prefix_len, int gqa_group_size, int block_m, int block_n, int head_dim, int dtype,
              void* workspace, size_t workspace_bytes, hipStream_t stream, const int64_t* q_strides) {
@@ -2372,12 +2376,15 @@ int gen_impl(const void* q, const KvSource& kv, void* o, float* lse, const int32
   ga.q = q;
   ga.k = kv.k;
   ga.v = kv.v;
-  ga.row_ptr = row_ptr;
-  ga.col_idx = col_idx;
-  ga.blk_type = blk_type;
-  ga.payload = payload;
-  ga.offset = offset;
-  for (int i = 0; i < 5; ++i) ga.ms[i] = meta_seq_stride[i];
+  ga.row_ptr = tree.row_ptr;
+  ga.col_idx = tree.col_idx;
+  ga.blk_type = tree.blk_type;
+  ga.payload = tree.payload;
+  ga.offset = tree.offset;
+  for (int i = 0; i < 5; ++i) ga.ms[i] = tree.seq_stride[i];
+  ga.mask = tree.mask;  // read by the kernel itself: no metadata needed
+  ga.mask_seq_stride = tree.n_masks > 1 ? tree.mask_seq_stride : 0;
+  ga.mask_row_stride = tree.mask_row_stride;
   ga.sqb = q_strides[0];
   ga.sqh = q_strides[1];
   ga.sqm = q_strides[2];
@@ -2458,14 +2465,10 @@ int fwd_impl(const void* q, const KvSource& kv, void* o, float* lse, const TreeS
   if (st != TSFA_OK) return st;
   for (int i = 0; i < 5; ++i)
     if (meta_seq_stride[i] < 0) return TSFA_ERR_INVALID_ARGUMENT;
-  if (gen_path(head_dim, dtype)) {
-    if (tree.mask != nullptr) st = tree.build(q_len, block_m, block_n, stream_);
-    if (st != TSFA_OK) return st;
-    return gen_impl(q, kv, o, lse, tree.row_ptr, tree.col_idx, tree.blk_type, tree.payload, tree.offset,
-                    meta_seq_stride, o_strides, sm_scale, batch, num_heads, num_kv_heads, q_len, kv_len, prefix_len,
+  if (gen_path(head_dim, dtype))
+    return gen_impl(q, kv, o, lse, tree, o_strides, sm_scale, batch, num_heads, num_kv_heads, q_len, kv_len, prefix_len,
                     gqa_group_size, block_m, block_n, head_dim, dtype, workspace, workspace_bytes,
                     reinterpret_cast<hipStream_t>(stream_), q_strides);
-  }
 
   // one snapshot of the TSFA_* switches for the whole call
   const Config cfg = config();

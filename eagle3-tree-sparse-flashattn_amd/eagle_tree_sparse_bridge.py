@@ -181,7 +181,7 @@ def _tree_call_plan(q, k, v, mask, block_m, block_n):
     _check_qkv(q, k, v)
     bsz, n_heads, q_len, head_dim = q.shape
     _, n_kv_heads, kv_len, _ = k.shape
-    if head_dim not in (64, 128) or not all(_layout_ok(t) for t in (q, k, v)):
+    if head_dim not in (64, 128, 256) or not all(_layout_ok(t) for t in (q, k, v)):
         return False
     if mask.dim() == 2:
         n_masks, seq_stride = 1, 0
@@ -212,7 +212,7 @@ def _tree_call(q, k, v, mask, block_m, block_n):
            block_n, q.device, (q.data_ptr() | k.data_ptr() | v.data_ptr()) & 15)
     entry = _TREE_CALLS.get(key)
     if entry is None:
-        if q.dtype not in (torch.float16, torch.bfloat16):
+        if q.dtype not in (torch.float16, torch.bfloat16, torch.float32):
             entry = False
         else:
             entry = _tree_call_plan(q, k, v, mask, block_m, block_n)

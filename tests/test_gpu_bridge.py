@@ -239,3 +239,25 @@ def test_mask_read_in_the_kernel_matches_the_metadata_route(b, hq, hkv, t, p, d,
         meta = bridge.build_tree_metadata(m, p, bm, bn)
         want = bridge.run_tree_sparse_kernel(q, k, v, None, block_m=bm, block_n=bn, metadata=meta)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# the generic kernel's mask read (words built in the prologue, and in the loop
+# for splits of more than 32 tree units) against its metadata route
+@pytest.mark.parametrize("dtype,b,hq,hkv,t,p,d", [
+    (torch.float32, 1, 4, 4, 128, 32, 64), (torch.float32, 2, 14, 2, 61, 77, 128), (torch.float32, 1, 2, 1, 9, 0, 256),
+    (torch.bfloat16, 3, 8, 2, 33, 100, 256), (torch.float16, 16, 64, 8, 1100, 65, 256),
+    (torch.float32, 16, 8, 8, 1061, 31, 64)])
+def test_generic_mask_read_matches_the_metadata_route(dtype, b, hq, hkv, t, p, d):
+    print(f"[bridge] generic mask read {dtype} b={b} hq={hq} hkv={hkv} t={t} p={p} d={d}", flush=True)
+    rng = np.random.default_rng(t)
+    masks = torch.from_numpy(np.stack([trees.ancestor_mask(trees.random_parents(t, rng)) for _ in range(b)])).cuda()
+    g = torch.Generator(device="cuda").manual_seed(t)
+    q, k, v = (torch.randn(s, generator=g, device="cuda").to(dtype)
+               for s in ((b, hq, t, d), (b, hkv, p + t, d), (b, hkv, p + t, d)))
+    for m in (masks, masks[0]):
+        bridge._TREE_CALLS.clear()
+        got = bridge.run_tree_sparse_kernel(q, k, v, m, block_m=64, block_n=64)
+        assert any(e is not False for e in bridge._TREE_CALLS.values())
+        meta = bridge.build_tree_metadata(m, p, 64, 64)
+        want = bridge.run_tree_sparse_kernel(q, k, v, None, block_m=64, block_n=64, metadata=meta)
+        assert torch.equal(got, want)
