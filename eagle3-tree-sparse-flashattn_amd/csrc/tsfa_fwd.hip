@@ -1850,8 +1850,7 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
   const int32_t* pl = a.payload + b * a.ms[3];
   const int32_t* of = a.offset + b * a.ms[4];
   const int qb = t / a.block_m, tl = t - qb * a.block_m;
-  const uint8_t* mrow = a.mask != nullptr ? a.mask + b * a.mask_seq_stride + t * a.mask_row_stride : nullptr;
-  const int e_lo = mrow != nullptr ? 0 : rp[qb], e_hi = mrow != nullptr ? 0 : rp[qb + 1];
+  const int e_lo = a.mask != nullptr ? 0 : rp[qb], e_hi = a.mask != nullptr ? 0 : rp[qb + 1];
   // Visibility of keys k0 .. k0+31 for the lane's row: prefix keys, then the
   // tree keys of the mask's row, or of the row's FULL and MIXED blocks (tree_sparse_flashattn.py:
   // 266-270, :307-318); keys past kv_len are not visible.
@@ -1860,8 +1859,8 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
     const int np = min(max(P - k0, 0), 32);
     uint32_t w = np >= 32 ? 0xffffffffu : ((1u << np) - 1u);
     const int c_lo = max(k0, P) - P, c_hi = min(k0 + 32, a.kv_len) - P;  // tree columns of the unit
-    if (c_lo < c_hi && mrow != nullptr) {
-      w |= mask_word(mrow, c_lo, a.kv_len - P) << (c_lo + P - k0);
+    if (c_lo < c_hi && a.mask != nullptr) {
+      w |= mask_word(a.mask + b * a.mask_seq_stride + t * a.mask_row_stride, c_lo, a.kv_len - P) << (c_lo + P - k0);
     } else if (c_lo < c_hi) {
       for (int e = e_lo; e < e_hi; ++e) {
         const int cb = ci[e] * BN;

@@ -57,15 +57,21 @@ __device__ inline uint32_t pack32(const uint8_t* p) {
   return word;
 }
 
-// Columns [c0, c0 + 32) of one mask row as bits, columns from n on 0 (c0 < n):
-// two vector loads, those of the row's cut last word ending at column n; the
-// byte loads are for rows of fewer than 32 columns.
+// Columns [c0, c0 + 32) of a mask row of n columns as bits, columns past its
+// end 0 (c0 < n, a multiple of 32).  A cut last word takes the 32 bytes that
+// end at column n; a row of fewer than 32 columns comes 8 bytes at a time (32
+// loads at once spill the fp32 head_dim 256 kernel).
 __device__ inline uint32_t mask_word(const uint8_t* row, int c0, int n) {
   const int valid = min(32, n - c0);
   if (c0 + valid >= 32) return pack32(row + c0 + valid - 32) >> (32 - valid);
   uint32_t word = 0;
+  for (int i0 = 0; i0 < n; i0 += 8) {
 #pragma unroll
-  for (int i = 0; i < 32; ++i) word |= (uint32_t)(i < valid && row[c0 + min(i, valid - 1)] != 0) << i;
+    for (int i = 0; i < 8; ++i) {
+      const int c = min(i0 + i, n - 1);  // past the end: the last byte again
+      word |= (uint32_t)(row[c] != 0) << c;
+    }
+  }
   return word;
 }
 

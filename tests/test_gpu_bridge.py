@@ -219,6 +219,7 @@ def test_one_call_path_refuses_kv_shorter_than_q():
 # the same units in the same order, so the same bits
 @pytest.mark.parametrize("b,hq,hkv,t,p,d,bm,bn", [
     (1, 4, 4, 1, 64, 64, 64, 64), (1, 4, 2, 7, 96, 128, 16, 16), (2, 8, 8, 31, 33, 64, 64, 48),
+    (2, 4, 2, 3, 96, 64, 16, 16), (1, 4, 4, 2, 64, 128, 16, 16), (1, 8, 2, 13, 96, 64, 16, 32), (1, 8, 2, 16, 64, 128, 16, 16),
     (3, 14, 2, 33, 1024, 64, 64, 64), (1, 32, 8, 61, 4095, 128, 16, 32), (16, 8, 2, 64, 2048, 128, 16, 64),
     (1, 8, 1, 200, 500, 128, 128, 128), (2, 4, 1, 95, 0, 128, 32, 64), (1, 4, 2, 1100, 640, 64, 16, 64),
     (1, 2, 2, 1200, 320, 128, 64, 64), (1, 8, 1, 515, 2048, 128, 1, 16)])
