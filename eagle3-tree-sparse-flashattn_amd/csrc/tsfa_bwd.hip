@@ -10,7 +10,7 @@
 // summed over the G query heads of each kv head.  P is recomputed from the
 // forward's per-row log-sum-exp (tsfa_fwd_lse).
 //
-// Kernels (one call = three or four launches, no host synchronisation):
+// Kernels (one call = two or three launches, no host synchronisation):
 //   * bwd_prep_vis_kernel, two jobs in one launch:
 //     prep -- per query row (16 lanes): Dv = rowsum(dO * O) in fp32, the
 //     log2-domain LSE, and (when the dQ pass is split) the row of the fp32 dQ
@@ -19,7 +19,7 @@
 //     P and dS are exactly 0;
 //     visibility -- per (32-row tile, tree key) a word (bit m: row 32*tile + m
 //     sees the key), from the CSR metadata;
-//   * bwd_kv_kernel (key-parallel, dK and dV): a workgroup owns 128 keys of
+//   * kv_role of bwd_main_kernel (key-parallel, dK and dV): a workgroup owns 128 keys of
 //     one (batch, kv head) -- prefix keys and tree keys in separate blocks --
 //     as 4 key groups x 2 row groups of waves; each wave keeps dK^T and dV^T
 //     of its 32 keys in registers while its row group walks every other
@@ -34,24 +34,21 @@
 //     copy of each tile serves both the row reads and the transposed reads
 //     (a swizzle that is conflict-free for both patterns).  The row groups
 //     merge their sums through LDS at the end;
-//   * bwd_dq_main_kernel (row-parallel, dQ): a workgroup owns 128 rows and a
-//     split of the 32-key units; S^T, dP^T, dS^T recomputed per unit and dQ^T
-//     += K^T dS^T accumulated in registers; an unsplit chunk writes dQ
+//   * dq_role of bwd_main_kernel (row-parallel, dQ): half a workgroup owns 128
+//     rows and a split of the 32-key units; S^T, dP^T, dS^T recomputed per unit
+//     and dQ^T += K^T dS^T accumulated in registers; an unsplit chunk writes dQ
 //     directly, split chunks add once per workgroup to the fp32 accumulator;
 //   * bwd_dq_kernel (split chunks only): dQ = sm_scale * accumulator in the
 //     input dtype.
-// bwd_kv_kernel and bwd_dq_main_kernel are independent once the first launch
-// has run; the dQ kernel goes to a side stream so its workgroups fill the CUs
-// the dK/dV grid leaves idle (70 -> 63 us per call at the Llama-3-8B shape,
-// where 264 dK/dV workgroups of one per CU leave a second round of 8).
+// The two roles are independent once the first launch has run; in one launch
+// the dQ workgroups fill the CUs that the dK / dV ones leave idle (264 of one
+// per CU at the Llama-3-8B shape: a second round of 8).
 
 #include <math.h>
 #include <stdlib.h>
 
 #include <algorithm>
 #include <atomic>
-#include <map>
-#include <mutex>
 #include <type_traits>
 #include <utility>
 
@@ -141,8 +138,11 @@ struct BwdArgs {
   float dq_scale;
   int dq_direct;
   int n_pu, n_tu;           // prefix / tree units of 32 keys
-  int n_chunks, n_splits, units_per_split, q_items, q_items_per_xcd;
+  int n_chunks, n_splits, units_per_split, q_items, q_pairs_per_xcd;
+  int first_block;  // of this launch (0, or the first dQ block when the passes run one after the other)
 };
+
+typedef __attribute__((address_space(4))) BwdArgs KArgs;  // in the kernel's argument segment
 
 template <int D> constexpr size_t kv_lds_bytes() {
   // K block | V block | 2 groups x kBufs x (Q tile, dO tile) | 2 x kBufs x 32 row stats |
@@ -169,8 +169,7 @@ template <int D> constexpr size_t kv_lds_bytes() {
 // load): 1.53 M -> 1.27 M cycles at that shape, 243 -> 105 VALU instructions
 // per 32 MFMAs.
 template <typename T, int D>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void bwd_kv_kernel(const BwdArgs a) {
+__device__ __forceinline__ void kv_role(const KArgs& a, const int blk, unsigned char* smem) {
   typedef typename Mma<T>::vec8 V8;
   constexpr int ROWB = D * 2;                 // bytes of one row
   constexpr int KSTEPS = D / 16;
@@ -185,7 +184,6 @@ void bwd_kv_kernel(const BwdArgs a) {
   static_assert(kBufs == 2, "the exchange at the end reuses the K, V and tile areas");
   static_assert(TPW >= 1 && KPW >= 1 && 2 * LPT == TPW * 4, "load split");
 
-  extern __shared__ __attribute__((aligned(256))) unsigned char smem[];  // tile bases keep bits 0-7 clear
   unsigned char* kblk = smem;
   unsigned char* vblk = kblk + KBLK_B;
   unsigned char* tiles = vblk + KBLK_B;  // group g, buffer s: Q at tiles + 2*(g*kBufs + s)*TILE_B, dO after
@@ -201,7 +199,7 @@ void bwd_kv_kernel(const BwdArgs a) {
   // XCD-aware item order: consecutive block ids go to different XCDs and each
   // XCD gets a contiguous item range, so the key blocks of one (b, kv head),
   // which read the same Q / dO tiles, share an L2.
-  const int item = (blockIdx.x & 7) * a.items_per_xcd + (blockIdx.x >> 3);
+  const int item = (blk & 7) * a.items_per_xcd + (blk >> 3);
   if (item >= a.n_items) return;
   const int nkb = a.n_pb + a.n_tb;
   const int kb = item % nkb;
@@ -486,7 +484,7 @@ template <int LPU, int K> __device__ inline void wait_units(int k) {
   }
 }
 
-// Row-parallel dQ: a workgroup owns a 128-row chunk of one (b, kv head) (one
+// Row-parallel dQ: half a workgroup owns a 128-row chunk of one (b, kv head) (one
 // 32-row tile per wave, Q and dO fragments in registers) and one split of its
 // 32-key units (prefix units, then the tree units), streamed through a
 // 4-stage LDS ring.  Per unit, on v_mfma_f32_32x32x16:
@@ -506,8 +504,7 @@ template <int LPU, int K> __device__ inline void wait_units(int k) {
 // offsets: 1.04 M -> 0.78 M cycles at that shape, 227 -> 88 VALU instructions
 // per 24 MFMAs.
 template <typename T, int D>
-__global__ __launch_bounds__(kQWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void bwd_dq_main_kernel(const BwdArgs a) {
+__device__ __forceinline__ void dq_role(const KArgs& a, const int blk, unsigned char* smem) {
   typedef typename Mma<T>::vec8 V8;
   constexpr int ROWB = D * 2;
   constexpr int KSTEPS = D / 16;
@@ -521,18 +518,19 @@ void bwd_dq_main_kernel(const BwdArgs a) {
   constexpr int UPW = 2 * LPH / kQWaves;   // K + V loads per wave per unit (wave 0 of a tree unit: one more)
   static_assert(UPW >= 1 && UPW * kQWaves == 2 * LPH && SB % 256 == 0, "load split, aligned stages");
 
-  extern __shared__ __attribute__((aligned(256))) unsigned char smem[];
-  unsigned char* ring = smem;
-
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = __builtin_amdgcn_readfirstlane(tid >> 8);
+  const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
+  unsigned char* ring = smem + half * kRing * SB;
   const int ln = lane & 31, lh = lane >> 5;
 
   // item order: chunk fastest (the chunks of one (b, kv head) read the same
   // K / V units), XCD-aware as in the forward
-  const int item = (blockIdx.x & 7) * a.q_items_per_xcd + (blockIdx.x >> 3);
-  if (item >= a.q_items) return;
+  const int pair = (blk & 7) * a.q_pairs_per_xcd + (blk >> 3);
+  if (2 * pair >= a.q_items) return;
+  const int item = min(2 * pair + half, a.q_items - 1);
+  const bool live = 2 * pair + half < a.q_items;
   const int chunk = item % a.n_chunks;
   int rest = item / a.n_chunks;
   const int sp = rest % a.n_splits;
@@ -544,11 +542,14 @@ void bwd_dq_main_kernel(const BwdArgs a) {
   const int P = a.prefix_len;
   const float sl2 = a.scale_log2;
   const int tile = chunk * kQWaves + wave;     // this wave's 32-row tile
-  const bool active = tile < a.n_tiles;
+  const bool active = live && tile < a.n_tiles;
   const int r = tile * kTileRows + ln;         // this lane's row
   const int n_units = a.n_pu + a.n_tu;
   const int u_lo = sp * a.units_per_split;
-  const int mine = max(0, min(a.units_per_split, n_units - u_lo));
+  const int mine = live ? max(0, min(a.units_per_split, n_units - u_lo)) : 0;
+  // steps of the workgroup: the longer half's (the halves share its barriers)
+  const int sp0 = (2 * pair) / a.n_chunks % a.n_splits, sp1 = min(2 * pair + 1, a.q_items - 1) / a.n_chunks % a.n_splits;
+  const int n_wg = min(a.units_per_split, n_units - min(sp0, sp1) * a.units_per_split);
 
   const T* kbase = static_cast<const T*>(a.k) + b * a.skb + kvh * a.skh;
   const T* vbase = static_cast<const T*>(a.v) + b * a.svb + kvh * a.svh;
@@ -746,6 +747,7 @@ void bwd_dq_main_kernel(const BwdArgs a) {
   } else {
     for (int j = 0; j < mine; ++j) step(j);
   }
+  for (int j = mine; j < n_wg; ++j) sync_lds();
   // lane (row ln, lh) holds d = dt*32 + 8(i/4) + 4lh + i%4.  One split per
   // chunk: the workgroup owns its rows' dQ and writes it in the input dtype.
   // Otherwise it adds to the d-major fp32 accumulator (each instruction's 64
@@ -775,6 +777,35 @@ void bwd_dq_main_kernel(const BwdArgs a) {
           atomicAdd(dq + (int64_t)(dt * 32 + 8 * (i >> 2) + (i & 3)) * TGP, acc[dt][i]);
     }
   }
+}
+
+// The two passes in one launch, dK / dV workgroups first (the longer ones),
+// so the dQ workgroups fill the CUs that their last round leaves idle.
+// Two launches, the second on a side stream forked and joined by events, cost
+// 46 us of host time per call against 10 us, so short training steps were
+// bound by it (8B shape, one layer's step: 196 -> 145 us), and the fork and
+// join on the device (its backward in a graph 59 -> 52 us; the 1024-token
+// tree's 1160 -> 991 with the loops above).  A dQ workgroup is two halves of
+// four waves with a row chunk and a ring each, as two workgroups per CU were.
+template <typename T, int D>
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void bwd_main_kernel(const BwdArgs a) {
+  extern __shared__ __attribute__((aligned(256))) unsigned char smem[];  // tile bases keep bits 0-7 clear
+  const int blk = blockIdx.x + a.first_block, n_kv = 8 * a.items_per_xcd;
+  // each role reads the arguments through a pointer of its own: loads hoisted
+  // above the branch for both spill SGPRs
+  const KArgs* ap = (const KArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  if (blk < n_kv) {
+    asm volatile("" : "+s"(ap));
+    kv_role<T, D>(*ap, blk, smem);
+  } else {
+    asm volatile("" : "+s"(ap));
+    dq_role<T, D>(*ap, blk - n_kv, smem);
+  }
+}
+
+template <int D> constexpr size_t main_lds_bytes() {
+  return kv_lds_bytes<D>() > 2 * dq_lds_bytes<D>() ? kv_lds_bytes<D>() : 2 * dq_lds_bytes<D>();
 }
 
 // ------------------------------------------------------------ prep / dq / vis
@@ -942,46 +973,6 @@ __global__ __launch_bounds__(256) void bwd_prep_vis_kernel(const PrepArgs pa, co
 }
 
 // ------------------------------------------------------------------- host
-// A side stream and fork/join events per (device, caller stream): the dQ
-// kernel runs beside the dK/dV kernel, so its workgroups fill the CUs that
-// the dK/dV grid leaves idle (a partial last round: 264 workgroups of one
-// per CU on 256 CUs at the Llama-3-8B shape).  Default priority; the side
-// stream does not synchronise with the null stream.  A call captured into a
-// graph forks and joins inside the capture.
-constexpr int kMaxSideStreams = 64;
-
-struct SideStream {
-  hipStream_t s = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
-};
-
-const SideStream* side_stream(hipStream_t stream) {
-  static std::mutex mu;
-  static std::map<std::pair<int, uintptr_t>, SideStream> sides;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-  std::lock_guard<std::mutex> lock(mu);
-  const auto key = std::make_pair(dev, reinterpret_cast<uintptr_t>(stream));
-  auto it = sides.find(key);
-  if (it != sides.end()) return &it->second;
-  // at most kMaxSideStreams per device; callers past that run on one stream
-  static int per_dev[64] = {};
-  if (dev < 0 || dev >= 64 || per_dev[dev] >= kMaxSideStreams) return nullptr;
-  SideStream ss;
-  if (hipStreamCreateWithFlags(&ss.s, hipStreamNonBlocking) != hipSuccess) return nullptr;
-  if (hipEventCreateWithFlags(&ss.fork, hipEventDisableTiming) != hipSuccess) {
-    (void)hipStreamDestroy(ss.s);
-    return nullptr;
-  }
-  if (hipEventCreateWithFlags(&ss.join, hipEventDisableTiming) != hipSuccess) {
-    (void)hipEventDestroy(ss.fork);
-    (void)hipStreamDestroy(ss.s);
-    return nullptr;
-  }
-  ++per_dev[dev];
-  return &sides.emplace(key, ss).first->second;
-}
-
 template <typename T, int D>
 int launch_bwd(const BwdArgs& ba, const PrepArgs& pa, const VisArgs& va, const DqArgs& da, const BwdPlan& p,
                bool has_tree, hipStream_t stream) {
@@ -990,11 +981,8 @@ int launch_bwd(const BwdArgs& ba, const PrepArgs& pa, const VisArgs& va, const D
   if (hipGetDevice(&dev) != hipSuccess) return TSFA_ERR_DEVICE;
   const uint64_t bit = 1ull << (dev & 63);
   if ((attr_set.load(std::memory_order_acquire) & bit) == 0) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_kv_kernel<T, D>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kv_lds_bytes<D>()) != hipSuccess)
-      return TSFA_ERR_LAUNCH;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dq_main_kernel<T, D>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)dq_lds_bytes<D>()) != hipSuccess)
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_main_kernel<T, D>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)main_lds_bytes<D>()) != hipSuccess)
       return TSFA_ERR_LAUNCH;
     attr_set.fetch_or(bit, std::memory_order_acq_rel);
   }
@@ -1006,23 +994,18 @@ int launch_bwd(const BwdArgs& ba, const PrepArgs& pa, const VisArgs& va, const D
   hipLaunchKernelGGL((bwd_prep_vis_kernel<T, D>), dim3((unsigned)(prep_blocks + vis_blocks)), dim3(256), 0, stream,
                      pa, va, (int)prep_blocks, std::max(1, vis_chunks));
   if (hipGetLastError() != hipSuccess) return TSFA_ERR_LAUNCH;
-  const unsigned grid = (unsigned)ba.items_per_xcd * 8;
-  const bool concurrent = config().bwd_concurrent != 0;  // TSFA_BWD_CONCURRENT=0: one stream (measurements)
-  const SideStream* side = (ba.q_items > 0 && concurrent) ? side_stream(stream) : nullptr;
-  if (side != nullptr && (hipEventRecord(side->fork, stream) != hipSuccess ||
-                          hipStreamWaitEvent(side->s, side->fork, 0) != hipSuccess))
+  auto launch_main = [&](int first, int blocks) {
+    BwdArgs a = ba;
+    a.first_block = first;
+    if (blocks > 0)
+      hipLaunchKernelGGL((bwd_main_kernel<T, D>), dim3((unsigned)blocks), dim3(kWaves * 64), main_lds_bytes<D>(),
+                         stream, a);
+    return hipGetLastError() == hipSuccess;
+  };
+  // TSFA_BWD_CONCURRENT=0: one pass after the other (measurements)
+  const int n_kv = ba.items_per_xcd * 8, n_dq = ba.q_pairs_per_xcd * 8;
+  if (config().bwd_concurrent != 0 ? !launch_main(0, n_kv + n_dq) : !launch_main(0, n_kv) || !launch_main(n_kv, n_dq))
     return TSFA_ERR_LAUNCH;
-  hipLaunchKernelGGL((bwd_kv_kernel<T, D>), dim3(grid), dim3(kWaves * 64), kv_lds_bytes<D>(), stream, ba);
-  if (hipGetLastError() != hipSuccess) return TSFA_ERR_LAUNCH;
-  if (ba.q_items > 0) {
-    const unsigned qgrid = (unsigned)ba.q_items_per_xcd * 8;
-    hipLaunchKernelGGL((bwd_dq_main_kernel<T, D>), dim3(qgrid), dim3(kQWaves * 64), dq_lds_bytes<D>(),
-                       side != nullptr ? side->s : stream, ba);
-    if (hipGetLastError() != hipSuccess) return TSFA_ERR_LAUNCH;
-    if (side != nullptr && (hipEventRecord(side->join, side->s) != hipSuccess ||
-                            hipStreamWaitEvent(stream, side->join, 0) != hipSuccess))
-      return TSFA_ERR_LAUNCH;
-  }
   if (ba.dq_direct) return TSFA_OK;
   const int64_t dq_threads = (int64_t)da.batch * da.num_kv_heads * da.q_len * da.group * (D / 8);
   hipLaunchKernelGGL((bwd_dq_kernel<T, D>), dim3((unsigned)((dq_threads + 255) / 256)), dim3(256), 0, stream, da);
@@ -1189,7 +1172,7 @@ extern "C" int tsfa_bwd(const void* q, const void* k, const void* v, const void*
     const int64_t q_items = n_units > 0 ? base * ba.n_splits : 0;
     if (q_items > INT32_MAX / 2) return TSFA_ERR_UNSUPPORTED;
     ba.q_items = (int)q_items;
-    ba.q_items_per_xcd = (ba.q_items + 7) / 8;
+    ba.q_pairs_per_xcd = ((ba.q_items + 1) / 2 + 7) / 8;
   }
   ba.dq = dq;
   ba.sdqb = strides[20];

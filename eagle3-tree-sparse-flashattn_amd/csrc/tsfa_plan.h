@@ -51,7 +51,7 @@ struct Config {
   int item_order;      // TSFA_ITEM_ORDER: 0/1/2 forces, -1 planner
   int paged32;         // TSFA_PAGED32: 0 keeps the 64-bit-offset paged kernel
   int meta_small;      // TSFA_META_SMALL: 0 always two metadata launches
-  int bwd_concurrent;  // TSFA_BWD_CONCURRENT: 0 keeps the backward on one stream
+  int bwd_concurrent;  // TSFA_BWD_CONCURRENT: 0 runs the backward's two passes one after the other
   int bench_hooks;     // TSFA_BENCH_HOOKS: 1 unlocks tsfa_fwd_set_kernel_mask
   int generation;      // bumped by every reload (keys of memoised plans)
 };

@@ -223,8 +223,7 @@ def test_bwd_graph_capture_replays():
 
 
 def test_bwd_two_streams_at_once(monkeypatch):
-    # each caller stream gets its own side stream for the dQ kernel: two
-    # backward calls in flight on two streams give the single-stream results
+    # two backward calls in flight on two streams give the single-stream results
     b, hq, hkv, t, p, d = 1, 32, 8, 64, 1024, 128
     mask = torch.from_numpy(_tree("eagle", t, np.random.default_rng(5)))
     meta = tsf.prepare_tree_sparse_metadata(mask.cuda(), p, 16, 64)
