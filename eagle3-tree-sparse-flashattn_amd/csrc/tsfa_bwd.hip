@@ -464,7 +464,6 @@ __device__ __forceinline__ void kv_role(const KArgs& a, const int blk, unsigned 
 // ------------------------------------------------------------- dQ kernel
 constexpr int kQWaves = 4;   // 32 rows each: 128-row chunks
 constexpr int kRing = 4;     // LDS ring stages of 32-key units
-constexpr int kMaxDqSplits = 16;
 
 template <int D> constexpr size_t dq_lds_bytes() {
   // kRing x (K unit, V unit, mask words of the chunk's 4 row tiles x 32 keys, padded to 256 bytes)
@@ -1153,10 +1152,9 @@ extern "C" int tsfa_bwd(const void* q, const void* k, const void* v, const void*
   ba.n_tkeys = p.n_tkeys;
   ba.n_items = batch * num_kv_heads * (p.n_pb + p.n_tb);
   // row-parallel dQ: 128-row chunks; the 32-key units (prefix, then the tree
-  // keys up to tree_key_limit) split so the grid covers about two workgroups
-  // per CU (two fit, and their waves interleave), at most kMaxDqSplits ways
-  // (each split adds its chunk's dQ once with atomics: splits x rows x D x 4
-  // bytes of atomic traffic; an unsplit chunk writes dQ directly)
+  // keys up to tree_key_limit) split by dq_splits (each split adds its chunk's
+  // dQ once with atomics: splits x rows x D x 4 bytes of atomic traffic; an
+  // unsplit chunk writes dQ directly)
   ba.n_pu = ceil_div(prefix_len, 32);
   ba.n_tu = ceil_div(tree_key_limit, 32);
   ba.n_chunks = ceil_div(p.n_tiles, kQWaves);
@@ -1165,8 +1163,8 @@ extern "C" int tsfa_bwd(const void* q, const void* k, const void* v, const void*
     if (device_cu_count(&cus) != TSFA_OK) return TSFA_ERR_DEVICE;
     const int n_units = ba.n_pu + ba.n_tu;
     const int64_t base = (int64_t)batch * num_kv_heads * ba.n_chunks;
-    const int64_t want = std::min<int64_t>(kMaxDqSplits, std::max<int64_t>(1, (2 * cus + base - 1) / base));
-    int splits = (int)std::min<int64_t>(want, std::max(1, n_units));
+    const int splits = n_units > 0 ? dq_splits(ba.n_items, (p.n_tiles + 1) / 2, base, n_units, head_dim,
+                                               (int64_t)p.dq_bytes, cus) : 1;
     ba.units_per_split = std::max(1, ceil_div(n_units, splits));
     ba.n_splits = std::max(1, ceil_div(n_units, ba.units_per_split));
     const int64_t q_items = n_units > 0 ? base * ba.n_splits : 0;
