@@ -1787,6 +1787,8 @@ constexpr int kGenStages(int stage_bytes) {
   return 131072 / stage_bytes < 2 ? 2 : (131072 / stage_bytes > 4 ? 4 : 131072 / stage_bytes);
 }
 
+constexpr int kGenPre = 1;  // units requested beside Q (at most NSTG - 1)
+
 template <typename T, int D, bool TW>
 __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs a) {
   constexpr bool F32 = std::is_same<T, float>::value;
@@ -1807,7 +1809,7 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
   // 128*(dt/EPL) + EPL*m + dt%EPL (m = 0..31)
   constexpr int EPL = D / 32 < 4 ? D / 32 : 4;
   static_assert(CPR >= 16 && LPW >= 1 && LPW * (NSTG - 2) < 64 && SB % (1024 * NW) == 0, "generic ring");
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  extern __shared__ __attribute__((aligned(256))) unsigned char smem[];  // stage bases keep bits 0-7 clear
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1910,10 +1912,6 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
       dma16(dbase + key * dstride + col, st + (uint32_t)i * 1024u);
     }
   };
-  // LDS byte offset of chunk c (16 B) of key row k within the K / V tile
-  auto swz = [](int k, int c) { return k * ROWB + ((c ^ (k & SWZ)) << 4); };
-  auto swv = [](int k, int c) { return k * ROWB + ((c ^ ((k & SWV) << 2)) << 4); };
-
   f32x16 o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -1929,43 +1927,27 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
   const int nt = max(0, u_lo + n - ut0);
   uint32_t* tw = reinterpret_cast<uint32_t*>(smem + NSTG * SB);
 
-  // ring prologue: Q (compiler-tracked loads, consumed here so the compiler's
-  // own waits never count the ring's), the first NSTG - 1 units, and with TW
-  // the tree words (their loads land behind the units')
-  for (int j = 0; j < NSTG - 1 && j < n; ++j) issue(j);
-  if constexpr (TW) {
-    for (int i = 0; i < nt; ++i) {
-      const uint32_t w = row_ok ? vis_word((ut0 + i) * 32) : 0u;
-      if (lh == 0 && dh == 0) tw[i * kGenRows + rg * 32 + ln] = w;
-    }
-  }
-  vm_wait<0>();
-#pragma unroll
-  for (int kk = 0; kk < KS; ++kk) asm volatile("" : : "v"(qf[kk]));
-  for (int j = 0; j < n; ++j) {
-    // unit j landed for every wave; stage (j - 1) % NSTG is free
-    wait_units<LPW, NSTG - 2>(min(n - 1 - j, NSTG - 2));
-    sync_lds();
-    if (j + NSTG - 1 < n) issue(j + NSTG - 1);
-    const unsigned char* kt = smem + (j % NSTG) * SB;
-    const unsigned char* vt = kt + TILE;
-    const int k0 = (u_lo + j) * 32;
-    // S^T: MFMA row = key, column = query row; lane (ln, lh) element i is key
-    // 8*(i/4) + 4*lh + i%4 of row ln
-    // (K read KA k-steps ahead of its MFMA, fenced: left to itself the
-    // scheduler reads one step ahead and every MFMA waits an LDS latency)
+  // S^T of the unit in stage kt: MFMA row = key, column = query row; lane (ln,
+  // lh) element i is key 8*(i/4) + 4*lh + i%4 of row ln.  K is read KA reads
+  // ahead of its MFMA, fenced (left to itself the scheduler reads one step
+  // ahead and every MFMA waits an LDS latency); between() runs after the first
+  // reads, slice(kk) after the MFMAs of read kk.
+  auto s_unit = [&](const unsigned char* kt, auto between, auto slice) {
     f32x16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
     constexpr int KA = F32 ? 2 : 4;
     QF kf[KS];
-    // fp32: read offsets formed anew each unit (hoisted out of the loop they
-    // spill the head_dim 256 instance)
-    int kr = ln;
-    if constexpr (F32) asm volatile("" : "+v"(kr));
-    auto rk = [&](int kk) { kf[kk] = *reinterpret_cast<const QF*>(kt + swz(kr, 2 * kk + lh)); };
+    // chunk 2kk + lh of key row ln: kk moves offset bits 5-7 under the XOR (one
+    // base register per unit; 16 hoisted offsets spill) and 256s past them
+    const uint32_t kb = lds_addr(kt) + (uint32_t)(ln * ROWB + ((lh ^ (ln & SWZ)) << 4));
+    auto rk = [&](int kk) {
+      kf[kk] = *(const TSFA_LDS QF*)((const TSFA_LDS char*)(uintptr_t)(kb ^ (uint32_t)((kk & 7) << 5)) + (kk >> 3) * 256);
+    };
 #pragma unroll
     for (int kk = 0; kk < KA; ++kk) rk(kk);
+    __builtin_amdgcn_sched_barrier(0);
+    between();
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk) {
       if (kk + KA < KS) rk(kk + KA);
@@ -1975,51 +1957,88 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
       } else {
         s = Mma<T>::run(bit_cast<typename Mma<T>::vec8>(kf[kk]), bit_cast<typename Mma<T>::vec8>(qf[kk]), s);
       }
+      slice(kk);
       __builtin_amdgcn_sched_barrier(0);
     }
-    // mask (units with a tree column only: every key of the others is a
-    // visible prefix key), online softmax (tree_sparse_flashattn.py:272-279,
-    // :320-327)
-    if (u_lo + j >= ut0) {
-      uint32_t w;
-      if constexpr (TW) w = tw[(u_lo + j - ut0) * kGenRows + rg * 32 + ln];
-      else w = row_ok ? vis_word(k0) : 0u;
+    return s;
+  };
+
+  // Unit j of the run (s: its S^T): mask, online softmax and O^T += V^T P^T;
+  // with NEXT, the S^T MFMAs of unit j + 1 (left in s) run with the
+  // exponentials of unit j between them.
+  auto unit = [&](auto next_c, int j, f32x16& s) {
+    constexpr bool NEXT = decltype(next_c)::value;
+    const unsigned char* vt = smem + (j % NSTG) * SB + TILE;
+    float alpha, ms;
+    bool need;
+    auto stats = [&]() {
+      // mask (units with a tree column only: every key of the others is a
+      // visible prefix key), online softmax (tree_sparse_flashattn.py:272-279,
+      // :320-327)
+      if (u_lo + j >= ut0) {
+        uint32_t w;
+        if constexpr (TW) w = tw[(u_lo + j - ut0) * kGenRows + rg * 32 + ln];
+        else w = row_ok ? vis_word((u_lo + j) * 32) : 0u;
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (!((w >> (8 * (i >> 2) + 4 * lh + (i & 3))) & 1u)) s[i] = -INFINITY;
-    }
-    float mx = -INFINITY;
+        for (int i = 0; i < 16; ++i)
+          if (!((w >> (8 * (i >> 2) + 4 * lh + (i & 3))) & 1u)) s[i] = -INFINITY;
+      }
+      float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-    const float rmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-    // The reference point m_run moves only when a score passes it by more
-    // than 2^kRescaleLog2 (or on the row's first visible key: m_lim is -inf
-    // until then), so p <= 2^8 and O is rescaled on few units: with 32 rows
-    // per wave some row's exact maximum moves on almost every unit, and each
-    // rescale moves the D / 2 accumulators of a lane through the VALU.
-    // Exact for any consistent reference point (tree_sparse_flashattn.py:
-    // 272-279 rescales at every block); a row that sees one key still gets
-    // p = 2^0 = 1, O = V bit for bit.
-    const bool need = rmax > m_lim;
-    const float m_new = need ? rmax : m_run;
-    // alpha = 0 on the first visible key (O and l are still 0)
-    const float alpha = need ? __builtin_amdgcn_exp2f((m_run - m_new) * sl2) : 1.f;
-    m_run = m_new;
-    m_lim = m_new + thr_raw;
-    // p = 2^((s - m_run) * scale); 0 for masked keys and while no key is visible
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      const float rmax = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      // The reference point m_run moves only when a score passes it by more
+      // than 2^kRescaleLog2 (or on the row's first visible key: m_lim is -inf
+      // until then), so p <= 2^8 and O is rescaled on few units: with 32 rows
+      // per wave some row's exact maximum moves on almost every unit, and each
+      // rescale moves the D / 2 accumulators of a lane through the VALU.
+      // Exact for any consistent reference point (tree_sparse_flashattn.py:
+      // 272-279 rescales at every block); a row that sees one key still gets
+      // p = 2^0 = 1, O = V bit for bit.
+      need = rmax > m_lim;
+      const float m_new = need ? rmax : m_run;
+      // alpha = 0 on the first visible key (O and l are still 0)
+      alpha = need ? __builtin_amdgcn_exp2f((m_run - m_new) * sl2) : 1.f;
+      m_run = m_new;
+      m_lim = m_new + thr_raw;
+      ms = m_new == -INFINITY ? 0.f : m_new;  // no key visible yet: every score is -inf
+    };
+    // p = 2^((s - m_run) * scale), 16-bit pairs of it rounded to the input
+    // dtype (tree_sparse_flashattn.py:278); 0 for masked keys (pinned where
+    // they are computed: the compiler sinks them past the re-base branch
+    // otherwise)
+    typedef T T2 __attribute__((ext_vector_type(2)));
     float p[16], ps = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      p[i] = (m_new == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((s[i] - m_new) * sl2);
+    uint32_t pk[8];
+    auto expo = [&](int i) {
+      p[i] = __builtin_amdgcn_exp2f((s[i] - ms) * sl2);
       ps += p[i];
+      if constexpr (F32) {
+        asm volatile("" : "+v"(p[i]), "+v"(ps));
+      } else if (i & 1) {
+        pk[i >> 1] = bit_cast<uint32_t>(T2{(T)p[i - 1], (T)p[i]});
+        asm volatile("" : "+v"(pk[i >> 1]), "+v"(ps));
+      }
+    };
+    if constexpr (NEXT) {
+      constexpr int EPK = KS < 16 ? 16 / KS : 1;  // exponentials after each K read's MFMAs
+      const f32x16 sn = s_unit(smem + ((j + 1) % NSTG) * SB, stats, [&](int kk) {
+#pragma unroll
+        for (int i = EPK * kk; i < EPK * (kk + 1) && i < 16; ++i) expo(i);
+      });
+      s = sn;
+    } else {
+      stats();
+#pragma unroll
+      for (int i = 0; i < 16; ++i) expo(i);
     }
     l_run = l_run * alpha + ps;
     if (__ballot(need) != 0) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
     }
-    // O^T += V^T P^T, P rounded to the input dtype (tree_sparse_flashattn.py:278)
+    // O^T += V^T P^T
     if constexpr (F32) {
       // k-step i: keys 8*(i/4) + 4*k + i%4 (k = 0, 1), lane (ln, lh) gives its
       // element i of P^T and EPL words of V's row 8*(i/4) + 4*lh + i%4, one
@@ -2045,9 +2064,8 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
       }
     } else {
       typedef typename Mma<T>::vec8 V8;
-      V8 pb[2];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) pb[i >> 3][i & 7] = (T)p[i];
+      typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+      const V8 pb[2] = {bit_cast<V8>(U4{pk[0], pk[1], pk[2], pk[3]}), bit_cast<V8>(U4{pk[4], pk[5], pk[6], pk[7]})};
       // V^T fragments by the transposing LDS read: lane i of 16-lane group x
       // gets keys 16*s2 + 8*jj + 4*(x>>1) + [0,4) of d = 32*gt + 16*(x&1) + i,
       // gt = dh*DT + dt the d-tile (bytes 64*gt + 2*(16*(x&1) + 4*(i&3)) of the
@@ -2055,16 +2073,16 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
       const int vx = lane >> 4, vi = lane & 15;
       const int vrow = 4 * (vx >> 1) + (vi >> 2);
       const int vch = 2 * (vx & 1) + ((vi & 3) >> 1), vhalf = 8 * (vi & 1);
+      static_assert(DT == 4, "a wave's d-tiles span two chunk bits");
+      const uint32_t vb = lds_addr(vt) + (uint32_t)(vrow * ROWB + ((vch ^ ((vrow & SWV) << 2)) << 4) + vhalf + dh * 256);
       // P V MFMA g = (dt, s2) = (g / 2, g % 2), its V^T read VA MFMAs ahead
       constexpr int NPV = 2 * DT, VA = 3;
       i16x4 vh[NPV][2];
       auto rv = [&](int g) {
-        const int dt = g >> 1, s2 = g & 1;
-        const int k0r = 16 * s2 + vrow, k1r = 16 * s2 + 8 + vrow;
-        vh[g][0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (TSFA_LDS i16x4*)(vt + swv(k0r, 4 * (dh * DT + dt) + vch) + vhalf));
-        vh[g][1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (TSFA_LDS i16x4*)(vt + swv(k1r, 4 * (dh * DT + dt) + vch) + vhalf));
+        // (d-tile dt moves offset bits 6-7 under the XOR; rows 8 apart share it)
+        const TSFA_LDS char* at = (const TSFA_LDS char*)(uintptr_t)(vb ^ (uint32_t)((g >> 1) << 6));
+        vh[g][0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TSFA_LDS i16x4*)(at + 16 * (g & 1) * ROWB));
+        vh[g][1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TSFA_LDS i16x4*)(at + (16 * (g & 1) + 8) * ROWB));
       };
 #pragma unroll
       for (int g = 0; g < VA && g < NPV; ++g) rv(g);
@@ -2075,6 +2093,52 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
         o[g >> 1] = Mma<T>::run(bit_cast<V8>(vf), pb[g & 1], o[g >> 1]);
         __builtin_amdgcn_sched_barrier(0);
       }
+    }
+  };
+
+  // Ring prologue: Q (compiler-tracked loads) leaves with the first kGenPre
+  // units and, with TW, the tree words; the rest of the ring is requested
+  // once they landed.  Every workgroup starts at once, so units requested
+  // beside Q queue ahead of other workgroups' Q in HBM (two units
+  // instead of one: 8 sequences behind 2k keys at head_dim 256 70.8
+  // against 69.7 us, the others within 0.5 us either way).
+  for (int j = 0; j < kGenPre && j < n; ++j) issue(j);
+  if constexpr (TW) {
+    for (int i = 0; i < nt; ++i) {
+      const uint32_t w = row_ok ? vis_word((ut0 + i) * 32) : 0u;
+      if (lh == 0 && dh == 0) tw[i * kGenRows + rg * 32 + ln] = w;
+    }
+  }
+  vm_wait<0>();
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk) asm volatile("" : : "v"(qf[kk]));
+  sync_lds();
+  for (int j = kGenPre; j < NSTG - 1 && j < n; ++j) issue(j);
+  auto no_op = [] {};
+  auto no_slice = [](int) {};
+  if constexpr (NSTG >= 3) {
+    // Iteration j reads V of unit j and K of unit j + 1: a wave's matrix core
+    // runs while its softmax does, and the first reads of K leave before the
+    // row maxima (with the ring's opening above, graph of calls: head_dim 256
+    // 8B decode shape 33.5 -> 31.1 us, 8 sequences behind 2k keys 76.0 -> 69.7,
+    // 512 tokens behind 8k 252 -> 242; fp32 8B shape 58.3 -> 56.8).
+    f32x16 s = s_unit(smem, no_op, no_slice);
+    for (int j = 0; j + 1 < n; ++j) {
+      // unit j + 1 landed for every wave; stage (j - 1) % NSTG is free
+      wait_units<LPW, NSTG - 3>(min(n - 2 - j, NSTG - 3));
+      sync_lds();
+      if (j + NSTG - 1 < n) issue(j + NSTG - 1);
+      unit(std::true_type{}, j, s);
+    }
+    unit(std::false_type{}, n - 1, s);
+  } else {
+    // two stages (fp32 head_dim 256): K of unit j + 1 lands while unit j runs
+    for (int j = 0; j < n; ++j) {
+      vm_wait<0>();
+      sync_lds();
+      if (j + 1 < n) issue(j + 1);
+      f32x16 s = s_unit(smem + (j % NSTG) * SB, no_op, no_slice);
+      unit(std::false_type{}, j, s);
     }
   }
 
