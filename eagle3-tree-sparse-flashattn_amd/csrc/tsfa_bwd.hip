@@ -139,7 +139,8 @@ struct BwdArgs {
   int dq_direct;
   int n_pu, n_tu;           // prefix / tree units of 32 keys
   int n_chunks, n_splits, units_per_split, q_items, q_pairs_per_xcd;
-  int first_block;  // of this launch (0, or the first dQ block when the passes run one after the other)
+  int dq_first;     // dQ workgroups before the dK / dV ones
+  int first_block;  // of this launch (0, or the second pass's first block when they run one after the other)
 };
 
 typedef __attribute__((address_space(4))) BwdArgs KArgs;  // in the kernel's argument segment
@@ -778,8 +779,8 @@ __device__ __forceinline__ void dq_role(const KArgs& a, const int blk, unsigned 
   }
 }
 
-// The two passes in one launch, dK / dV workgroups first (the longer ones),
-// so the dQ workgroups fill the CUs that their last round leaves idle.
+// The two passes in one launch, so the second one's workgroups fill the CUs
+// that the first one's last round leaves idle (dq_split_plan: which is first).
 // Two launches, the second on a side stream forked and joined by events, cost
 // 46 us of host time per call against 10 us, so short training steps were
 // bound by it (8B shape, one layer's step: 196 -> 145 us), and the fork and
@@ -790,16 +791,18 @@ template <typename T, int D>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_main_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(256))) unsigned char smem[];  // tile bases keep bits 0-7 clear
-  const int blk = blockIdx.x + a.first_block, n_kv = 8 * a.items_per_xcd;
+  const int id = blockIdx.x + a.first_block;
+  const int n_first = 8 * (a.dq_first ? a.q_pairs_per_xcd : a.items_per_xcd);
+  const int blk = id < n_first ? id : id - n_first;
   // each role reads the arguments through a pointer of its own: loads hoisted
   // above the branch for both spill SGPRs
   const KArgs* ap = (const KArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-  if (blk < n_kv) {
+  if ((id < n_first) != (a.dq_first != 0)) {
     asm volatile("" : "+s"(ap));
     kv_role<T, D>(*ap, blk, smem);
   } else {
     asm volatile("" : "+s"(ap));
-    dq_role<T, D>(*ap, blk - n_kv, smem);
+    dq_role<T, D>(*ap, blk, smem);
   }
 }
 
@@ -1006,8 +1009,9 @@ int launch_bwd(const BwdArgs& ba, const PrepArgs& pa, const VisArgs& va, const D
     return hipGetLastError() == hipSuccess;
   };
   // TSFA_BWD_CONCURRENT=0: one pass after the other (measurements)
-  const int n_kv = ba.items_per_xcd * 8, n_dq = ba.q_pairs_per_xcd * 8;
-  if (config().bwd_concurrent != 0 ? !launch_main(0, n_kv + n_dq) : !launch_main(0, n_kv) || !launch_main(n_kv, n_dq))
+  const int n1 = 8 * (ba.dq_first ? ba.q_pairs_per_xcd : ba.items_per_xcd);
+  const int n2 = 8 * (ba.dq_first ? ba.items_per_xcd : ba.q_pairs_per_xcd);
+  if (config().bwd_concurrent != 0 ? !launch_main(0, n1 + n2) : !launch_main(0, n1) || !launch_main(n1, n2))
     return TSFA_ERR_LAUNCH;
   if (ba.dq_direct) return TSFA_OK;
   const int64_t dq_threads = (int64_t)da.batch * da.num_kv_heads * da.q_len * da.group * (D / 8);
@@ -1156,7 +1160,7 @@ extern "C" int tsfa_bwd(const void* q, const void* k, const void* v, const void*
   ba.n_tkeys = p.n_tkeys;
   ba.n_items = batch * num_kv_heads * (p.n_pb + p.n_tb);
   // row-parallel dQ: 128-row chunks; the 32-key units (prefix, then the tree
-  // keys up to tree_key_limit) split by dq_splits (each split adds its chunk's
+  // keys up to tree_key_limit) split by dq_split_plan (each split adds its chunk's
   // dQ once with atomics: splits x rows x D x 4 bytes of atomic traffic; an
   // unsplit chunk writes dQ directly)
   ba.n_pu = ceil_div(prefix_len, 32);
@@ -1167,8 +1171,12 @@ extern "C" int tsfa_bwd(const void* q, const void* k, const void* v, const void*
     if (device_cu_count(&cus) != TSFA_OK) return TSFA_ERR_DEVICE;
     const int n_units = ba.n_pu + ba.n_tu;
     const int64_t base = (int64_t)batch * num_kv_heads * ba.n_chunks;
-    const int splits = n_units > 0 ? dq_splits(ba.n_items, (p.n_tiles + 1) / 2, base, n_units, head_dim,
-                                               (int64_t)p.dq_bytes, cus) : 1;
+    int splits = 1;
+    bool dq_first = false;
+    if (n_units > 0)
+      dq_split_plan(ba.n_items, (p.n_tiles + 1) / 2, base, n_units, head_dim, (int64_t)p.dq_bytes, cus, &splits,
+                    &dq_first);
+    ba.dq_first = dq_first ? 1 : 0;
     ba.units_per_split = std::max(1, ceil_div(n_units, splits));
     ba.n_splits = std::max(1, ceil_div(n_units, ba.units_per_split));
     const int64_t q_items = n_units > 0 ? base * ba.n_splits : 0;

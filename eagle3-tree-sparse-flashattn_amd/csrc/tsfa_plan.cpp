@@ -319,42 +319,58 @@ int make_bwd_plan(int batch, int num_kv_heads, int q_len, int kv_len, int prefix
   return TSFA_OK;
 }
 
-// The split count with the earliest modelled end of the launch.  Workgroups
-// take one CU each, dK / dV first: a dK / dV item takes 8.2 us + 1.71 us per
-// step, a dQ item (two chunk splits side by side) 10 us + 1.36 us per unit (at
-// head_dim 128, fitted on MI355X), and the accumulator's atomics 2 TB/s.  What
-// decides is how the dQ items fill the CUs that the last dK / dV round leaves:
-// with two workgroups per CU aimed at instead, whatever the round (backward
-// alone): 100 tokens of 8 heads behind 16k keys 10 splits 286 us, 8 243 us;
-// 700 tokens, one head per kv head, 11 splits 64 us, 3 60.5; the 16-sequence
-// shape 1 or 2 splits 220 us, 4 236.
-int dq_splits(int64_t kv_items, int steps, int64_t chunks, int n_units, int head_dim, int64_t acc_bytes, int cus) {
+namespace {
+// End of a launch of `na` workgroups of `a` us each, then `nb` of `b` us, one
+// per CU at a time, dispatched in order.
+double launch_end(int64_t na, double a, int64_t nb, double b, int cus) {
+  const int64_t last = na % cus;                // CUs with one of the first kind more
+  const double t1 = (double)(na / cus) * a;     // the others are free here
+  const double first_end = last > 0 ? t1 + a : t1;
+  if (nb > 32 * (int64_t)cus)
+    return std::max(first_end, (t1 * (cus - last) + (t1 + a) * last + b * nb) / cus + 0.5 * b);
+  double end = first_end, x = t1 + b, y = t1 + a + b;  // next end on either kind of CU
+  for (int64_t done = 0; done < nb;) {
+    if (last == 0 || x <= y) {
+      end = std::max(end, x), done += cus - last, x += b;
+    } else {
+      end = std::max(end, y), done += last, y += b;
+    }
+  }
+  return end;
+}
+}  // namespace
+
+// The split count and dispatch order with the earliest modelled end of the
+// launch.  Workgroups take one CU each: a dK / dV item takes 8.2 us + 1.71 us
+// per step, a dQ item (two chunk splits side by side) 10 us + 1.36 us per unit
+// (at head_dim 128, fitted on MI355X), and the accumulator's atomics 2 TB/s.
+// What decides is how the second kind fills the CUs that the first kind's last
+// round leaves: with two dQ workgroups per CU aimed at instead, behind the
+// dK / dV ones whatever the round (backward alone): 100 tokens of 8 heads
+// behind 16k keys 10 splits 286 us, 8 243 us; 700 tokens, one head per kv
+// head, 11 splits 64 us, 3 60.5; the 16-sequence shape 1 or 2 splits 220 us, 4
+// 236.  And with dQ first where that ends earlier, against dK / dV first
+// always: the 8B shape 52.0 -> 40.3 us, the 16-sequence shape 214 -> 176, 4
+// sequences behind 8k keys 314 -> 284, the 1024-token tree 970 -> 936.
+void dq_split_plan(int64_t kv_items, int steps, int64_t chunks, int n_units, int head_dim, int64_t acc_bytes,
+                   int cus, int* splits, bool* dq_first) {
   const double d = head_dim / 128.0;
   const double kv_us = 8.2 + 1.71 * d * steps;
-  const int64_t last = kv_items % cus;                 // CUs with one dK / dV round more
-  const double t1 = (double)(kv_items / cus) * kv_us;  // the others are free here
-  int best = 1;
   double best_us = 0;
+  *splits = 1;
+  *dq_first = false;
   for (int want = 1; want <= std::min(kMaxDqSplits, n_units); ++want) {
     const int units = ceil_div(n_units, want), s = ceil_div(n_units, units);
     if (s != want) continue;
     const double item = 10.0 + 1.36 * d * units;
     const int64_t items = (chunks * s + 1) / 2;
-    double end = (t1 * (cus - last) + (t1 + kv_us) * last + item * items) / cus + 0.5 * item;
-    if (items <= 32 * (int64_t)cus) {  // few rounds: where exactly they end
-      double a = t1 + item, b = t1 + kv_us + item;  // next end on either kind of CU
-      for (int64_t done = 0; done < items;) {
-        if (last == 0 || a <= b) {
-          end = a, done += cus - last, a += item;
-        } else {
-          end = b, done += last, b += item;
-        }
-      }
+    for (int order = 0; order < 2; ++order) {
+      const double end = (order == 0 ? launch_end(kv_items, kv_us, items, item, cus)
+                                     : launch_end(items, item, kv_items, kv_us, cus)) +
+                         (s > 1 ? (double)acc_bytes * s / 2e6 : 0.0);
+      if ((want == 1 && order == 0) || end < best_us) *splits = s, *dq_first = order == 1, best_us = end;
     }
-    if (s > 1) end += (double)acc_bytes * s / 2e6;
-    if (want == 1 || end < best_us) best = s, best_us = end;
   }
-  return best;
 }
 
 }  // namespace bwd

@@ -134,9 +134,11 @@ int make_bwd_plan(int batch, int num_kv_heads, int q_len, int kv_len, int prefix
 constexpr int kMaxDqSplits = 16;
 
 // Key splits of each of the dQ pass's `chunks` 128-row chunks (all groups
-// together), n_units 32-key units each, behind kv_items dK / dV workgroups of
-// `steps` tile pairs, on cus compute units; acc_bytes: the fp32 accumulator.
-int dq_splits(int64_t kv_items, int steps, int64_t chunks, int n_units, int head_dim, int64_t acc_bytes, int cus);
+// together), n_units 32-key units each, beside kv_items dK / dV workgroups of
+// `steps` tile pairs, on cus compute units (acc_bytes: the fp32 accumulator),
+// and whether they are dispatched first.
+void dq_split_plan(int64_t kv_items, int steps, int64_t chunks, int n_units, int head_dim, int64_t acc_bytes,
+                   int cus, int* splits, bool* dq_first);
 
 }  // namespace bwd
 
