@@ -58,9 +58,9 @@ __device__ inline uint32_t pack32(const uint8_t* p) {
 }
 
 // Columns [c0, c0 + 32) of a mask row of n columns as bits, columns past its
-// end 0 (c0 < n, a multiple of 32).  A cut last word takes the 32 bytes that
-// end at column n; a row of fewer than 32 columns comes 8 bytes at a time (32
-// loads at once spill the fp32 head_dim 256 kernel).
+// end 0 (c0 < n).  A cut last word takes the 32 bytes that end at column n; a
+// row of fewer than 32 columns comes whole, 8 bytes at a time (32 loads at
+// once spill the fp32 head_dim 256 kernel).
 __device__ inline uint32_t mask_word(const uint8_t* row, int c0, int n) {
   const int valid = min(32, n - c0);
   if (c0 + valid >= 32) return pack32(row + c0 + valid - 32) >> (32 - valid);
@@ -72,7 +72,7 @@ __device__ inline uint32_t mask_word(const uint8_t* row, int c0, int n) {
       word |= (uint32_t)(row[c] != 0) << c;
     }
   }
-  return word;
+  return word >> c0;
 }
 
 // ---------------------------------------------------------- host utilities

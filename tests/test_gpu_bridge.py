@@ -246,6 +246,7 @@ def test_mask_read_in_the_kernel_matches_the_metadata_route(b, hq, hkv, t, p, d,
 # for splits of more than 32 tree units) against its metadata route
 @pytest.mark.parametrize("dtype,b,hq,hkv,t,p,d", [
     (torch.float32, 1, 4, 4, 128, 32, 64), (torch.float32, 2, 14, 2, 61, 77, 128), (torch.float32, 1, 2, 1, 9, 0, 256),
+    (torch.float32, 3, 8, 2, 31, 2451, 128), (torch.bfloat16, 2, 4, 4, 20, 77, 256), (torch.float32, 1, 4, 2, 5, 30, 64),
     (torch.bfloat16, 3, 8, 2, 33, 100, 256), (torch.float16, 16, 64, 8, 1100, 65, 256),
     (torch.float32, 16, 8, 8, 1061, 31, 64)])
 def test_generic_mask_read_matches_the_metadata_route(dtype, b, hq, hkv, t, p, d):
