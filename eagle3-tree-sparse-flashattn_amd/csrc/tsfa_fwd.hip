@@ -1933,9 +1933,12 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
   // ahead and every MFMA waits an LDS latency); between() runs after the first
   // reads, slice(kk) after the MFMAs of read kk.
   auto s_unit = [&](const unsigned char* kt, auto between, auto slice) {
-    f32x16 s;
+    // fp32: two half sums (the odd K reads' apart) round less than one chain
+    // (head_dim 256 has no registers for it)
+    constexpr bool TWO = F32 && D <= 128;
+    f32x16 s, s1;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+    for (int i = 0; i < 16; ++i) s[i] = s1[i] = 0.f;
     constexpr int KA = F32 ? 2 : 4;
     QF kf[KS];
     // chunk 2kk + lh of key row ln: kk moves offset bits 5-7 under the XOR (one
@@ -1953,12 +1956,19 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
       if (kk + KA < KS) rk(kk + KA);
       if constexpr (F32) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[kk][e], qf[kk][e], s, 0, 0, 0);
+        for (int e = 0; e < 4; ++e) {
+          if (TWO && (kk & 1)) s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[kk][e], qf[kk][e], s1, 0, 0, 0);
+          else s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[kk][e], qf[kk][e], s, 0, 0, 0);
+        }
       } else {
         s = Mma<T>::run(bit_cast<typename Mma<T>::vec8>(kf[kk]), bit_cast<typename Mma<T>::vec8>(qf[kk]), s);
       }
       slice(kk);
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (TWO) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] += s1[i];
     }
     return s;
   };
