@@ -2207,12 +2207,12 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
 }
 
 // The generic kernel's plan: 128-row chunks, the key axis cut into n_slots
-// splits of whole 32-key units: about one workgroup per compute unit, with
-// the partials (written once, read once by the combine) held to at most
-// the K/V bytes or 8 MB, whichever is larger (the 8B decode shape at
-// head_dim 256 with fp32 partials: 16 splits, 36.8 us per call, against 40.5
-// with half the K/V bytes (8 splits, half the CUs idle); twice the K/V
-// bytes: the same 16).
+// splits of whole 32-key units: the count with the least modelled time over
+// the rounds of workgroups it makes, with the partials (written once, read
+// once by the combine) held to at most the K/V bytes or 8 MB, whichever is
+// larger (the 8B decode shape at head_dim 256 with fp32 partials: 16 splits,
+// 36.8 us per call, against 40.5 with half the K/V bytes (8 splits, half the
+// CUs idle); twice the K/V bytes: the same 16).
 struct GenPlan {
   int n_chunks, n_units, units_per_split, n_slots, grid;
   size_t lds_bytes, ws_acc_bytes, ws_ml_bytes;
@@ -2232,9 +2232,26 @@ inline int gen_plan(int batch, int num_heads, int num_kv_heads, int q_len, int k
   const size_t es = dtype == TSFA_DTYPE_FP32 ? 4 : 2;
   const double kv_bytes = 2.0 * batch * num_kv_heads * (double)kv_len * head_dim * es;
   const double slot_bytes = (double)batch * num_heads * q_len * ((double)es * head_dim + 8.0);
-  const int64_t want = std::max<int64_t>(1, ((int64_t)cus + groups - 1) / groups);
-  const int64_t cap = std::max<int64_t>(1, (int64_t)(std::max(kv_bytes, 8.0 * (1 << 20)) / slot_bytes));
-  const int slots = (int)std::min<int64_t>(p->n_units, std::min(want, cap));
+  int64_t cap = std::max<int64_t>(1, (int64_t)(std::max(kv_bytes, 8.0 * (1 << 20)) / slot_bytes));
+  // past one workgroup per CU only while the partials fit the allocation-free
+  // forward's array with room to spare
+  const int64_t fill = std::max<int64_t>(1, ((int64_t)cus + groups - 1) / groups);
+  cap = std::min(cap, std::max(fill, (int64_t)(0.75 * TSFA_FWD_NOALLOC_MAX_BYTES / slot_bytes)));
+  // One workgroup per CU, a unit's time and 8 us per workgroup, and with
+  // several splits the combine and the partials at 2 TB/s.  Splits aimed at
+  // one workgroup per CU instead left last rounds nearly empty: 168 groups at
+  // head_dim 256 (3 sequences of 200 tokens behind 3k keys) 2 splits 161 us, 3
+  // 139; 320 fp32 groups (2 of 300 tokens behind 1k keys) 214 -> 201.
+  const double unit_us = dtype == TSFA_DTYPE_FP32 ? 5.0 * head_dim / 128 : 1.9;
+  int slots = 1;
+  double best = 0;
+  for (int want = 1; want <= std::min<int64_t>(std::min(cap, (int64_t)cus), p->n_units); ++want) {
+    const int units = ceil_div(p->n_units, want), n = ceil_div(p->n_units, units);
+    if (n != want) continue;
+    const int64_t rounds = (groups * n + cus - 1) / cus;
+    const double us = (double)rounds * (8.0 + units * unit_us) + (n > 1 ? 5.0 + n * slot_bytes / 2e6 : 0.0);
+    if (want == 1 || us < best) slots = n, best = us;
+  }
   p->units_per_split = ceil_div(p->n_units, slots);
   p->n_slots = ceil_div(p->n_units, p->units_per_split);
   const int64_t grid = groups * p->n_slots;
