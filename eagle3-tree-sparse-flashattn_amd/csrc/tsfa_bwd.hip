@@ -1212,13 +1212,9 @@ extern "C" int tsfa_bwd(const void* q, const void* k, const void* v, const void*
   pa.zero_dq = ba.dq_direct ? 0 : 1;
   ba.group_magic = gqa_group_size > 1 ? (uint32_t)((((uint64_t)1) << 32) / (uint64_t)gqa_group_size + 1) : 0u;
   ba.items_per_xcd = (ba.n_items + 7) / 8;
-  // a tile's (unit's) lanes reach this far past its first token (key), in bytes
-  auto lane_reach = [&](int64_t sh, int64_t sm) {
-    return 2 * ((gqa_group_size - 1) * sh + (kTileRows / gqa_group_size - 1) * sm + head_dim);
-  };
-  ba.tile_fast = 32 % gqa_group_size == 0 && lane_reach(ba.sqh, ba.sqm) < INT32_MAX &&
-                 lane_reach(ba.sdoh, ba.sdom) < INT32_MAX;
-  ba.key_fast = 2 * (31 * std::max(ba.skn, ba.svn) + head_dim) < INT32_MAX;
+  ba.tile_fast = tile_offsets_fit(gqa_group_size, ba.sqh, ba.sqm, head_dim) &&
+                 tile_offsets_fit(gqa_group_size, ba.sdoh, ba.sdom, head_dim);
+  ba.key_fast = unit_offsets_fit(ba.skn, head_dim) && unit_offsets_fit(ba.svn, head_dim);
 
   DqArgs da;
   da.dq_acc = dq_acc;

@@ -319,6 +319,15 @@ int make_bwd_plan(int batch, int num_kv_heads, int q_len, int kv_len, int prefix
   return TSFA_OK;
 }
 
+bool tile_offsets_fit(int gqa, int64_t sh, int64_t sm, int head_dim) {
+  if (gqa <= 0 || kTileRows % gqa != 0 || sh < 0 || sm < 0 || sh > INT32_MAX || sm > INT32_MAX) return false;
+  return 2 * ((gqa - 1) * sh + (kTileRows / gqa - 1) * sm + head_dim) <= INT32_MAX;
+}
+
+bool unit_offsets_fit(int64_t sn, int head_dim) {
+  return sn >= 0 && sn <= INT32_MAX && 2 * (31 * sn + head_dim) <= INT32_MAX;
+}
+
 namespace {
 // End of a launch of `na` workgroups of `a` us each, then `nb` of `b` us, one
 // per CU at a time, dispatched in order.

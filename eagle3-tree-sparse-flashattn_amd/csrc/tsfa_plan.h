@@ -131,6 +131,14 @@ struct BwdPlan {
 int make_bwd_plan(int batch, int num_kv_heads, int q_len, int kv_len, int prefix_len, int gqa, int head_dim,
                   int block_m, int n_tree_blocks, int n_trees, BwdPlan* p);
 
+// Whether the 32-bit lane offsets of a whole 32-row Q / dO tile from its first
+// token (row r: (r % gqa) * sh + (r / gqa) * sm elements of 2 bytes, gqa
+// dividing 32), and of a whole 32-key K / V unit from its first key (sn
+// elements a key), stay in [0, 2^31): the loads add them unsigned, so a
+// negative stride takes the 64-bit addresses instead.
+bool tile_offsets_fit(int gqa, int64_t sh, int64_t sm, int head_dim);
+bool unit_offsets_fit(int64_t sn, int head_dim);
+
 constexpr int kMaxDqSplits = 16;
 
 // Key splits of each of the dQ pass's `chunks` 128-row chunks (all groups

@@ -192,6 +192,31 @@ static void sweep_bwd_plan() {
   }
 }
 
+// The backward's scalar-base loads: where the rule allows them, every lane
+// offset of a tile (unit), formed in 64 bits, is what 32 unsigned bits hold.
+static void sweep_bwd_offsets() {
+  for (int it = 0; it < 100000; ++it) {
+    const int gqa = (int)uni(1, 40), D = uni(0, 1) ? 64 : 128;
+    auto stride = [] { return 8 * (uni(0, 3) ? uni(-4096, 1 << 16) : uni(-(1ll << 57), 1ll << 57)); };
+    const int64_t sh = stride(), sm = stride();
+    if (bwd::tile_offsets_fit(gqa, sh, sm, D)) {
+      for (int row = 0; row < bwd::kTileRows; ++row) {
+        const int t = row / gqa;
+        const int64_t lo = ((row - t * gqa) * sh + t * sm) * 2, hi = lo + 2 * D;
+        EXPECT(lo >= 0 && hi <= (1ll << 31), "gqa %d sh %lld sm %lld", gqa, (long long)sh, (long long)sm);
+      }
+    }
+    if (bwd::unit_offsets_fit(sm, D))
+      for (int row = 0; row < 32; ++row)
+        EXPECT(row * sm >= 0 && 2 * (row * sm + D) <= (1ll << 31), "sn %lld", (long long)sm);
+  }
+  // dense and transposed 8B layouts take the scalar base, reversed ones do not
+  EXPECT(bwd::tile_offsets_fit(4, 64 * 128, 128, 128) && bwd::tile_offsets_fit(4, 128, 32 * 128, 128), "8B q");
+  EXPECT(!bwd::tile_offsets_fit(4, 64 * 128, -128, 128) && !bwd::tile_offsets_fit(4, -128, 4096, 128), "reversed q");
+  EXPECT(!bwd::tile_offsets_fit(7, 64 * 64, 64, 64), "7 query heads");
+  EXPECT(bwd::unit_offsets_fit(128, 128) && bwd::unit_offsets_fit(0, 128) && !bwd::unit_offsets_fit(-128, 128), "k");
+}
+
 static void sweep_meta() {
   for (int it = 0; it < 3000; ++it) {
     const int n_seq = (int)uni(1, 3), q_len = (int)uni(0, 90), bm = (int)uni(1, 40), bn = (int)uni(1, 40);
@@ -274,6 +299,7 @@ int main() {
   sweep_check_args();
   sweep_layouts();
   sweep_bwd_plan();
+  sweep_bwd_offsets();
   sweep_meta();
   if (g_fail) {
     fprintf(stderr, "%d invariant violations\n", g_fail);

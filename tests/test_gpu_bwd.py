@@ -19,7 +19,7 @@ import torch
 
 import tree_sparse_flashattn as tsf
 from oracle.attn_grad_oracle import attention_grads
-from tsfa import configs, trees
+from tsfa import _lib, configs, trees
 
 pytestmark = pytest.mark.gpu
 
@@ -249,3 +249,38 @@ def test_bwd_two_streams_at_once(monkeypatch):
         for dq, dk, dv in outs[j]:
             assert torch.equal(dk, refs[j][1]) and torch.equal(dv, refs[j][2])
             torch.testing.assert_close(dq, refs[j][0], rtol=1e-2, atol=1e-3)
+
+
+def test_bwd_reversed_rows_and_keys():
+    # the C entry takes negative strides: tokens of q and dO and keys of K and V
+    # stored last to first give the gradients of the dense call
+    b, hq, hkv, t, p, d = 1, 8, 2, 64, 200, 128
+    print("[bwd] reversed rows and keys", flush=True)
+    mask = torch.from_numpy(_tree("random", t, np.random.default_rng(8)))
+    q, k, v, do = (x.cuda() for x in _inputs(b, hq, hkv, t, p, d, BF, seed=8))
+    meta = tsf.prepare_tree_sparse_metadata(mask.cuda(), p, 16, 16)
+    o, lse = tsf.tree_sparse_attention_fwd(q, k, v, meta, return_lse=True)
+    want = tsf.tree_sparse_attention_bwd(q, k, v, o, lse, do, meta)
+    dq, dk, dv = (torch.full_like(x, float("nan")) for x in (q, k, v))
+    rev = [x.flip(2).contiguous() for x in (q, k, v, do)]  # kept alive over the call
+
+    def back(x):  # the view that reads x's dim 2 last to first: (first element, strides)
+        s = list(x.stride())
+        return x.data_ptr() + (x.shape[2] - 1) * s[2] * x.element_size(), (s[0], s[1], -s[2], s[3])
+
+    (qp, qs), (kp, ks), (vp, vs), (dop, dos) = (back(x) for x in rev)
+    lib = _lib.load()
+    args = (b, hq, hkv, t, p + t, p, meta.n_q_blocks, meta.n_tree_blocks, hq // hkv, 16, 16, d, _lib.dtype_code(BF))
+    ws_bytes = lib.tsfa_bwd_workspace_bytes(b, hq, hkv, t, p + t, p, 16, meta.n_tree_blocks, d, 1)
+    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device="cuda")
+    strides = (*qs, *ks, *vs, *o.stride(), *dos, *dq.stride(), *dk.stride(), *dv.stride())
+    st = lib.tsfa_bwd(qp, kp, vp, o.data_ptr(), lse.data_ptr(), dop, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                      *(_lib.ptr(x) for x in (meta.row_ptr, meta.col_idx, meta.blk_type, meta.mixed_mask_payload,
+                                              meta.mixed_mask_offset)),
+                      _lib.i64_array((0,) * 5), _lib.i64_array(strides), 1.0 / math.sqrt(d), *args, ws.data_ptr(),
+                      ws_bytes, _lib.stream_handle(q.device))
+    torch.cuda.synchronize()
+    assert st == _lib.TSFA_OK
+    assert torch.equal(dk, want[1]) and torch.equal(dv, want[2])
+    # dQ sums fp32 atomics of the key splits in a run-dependent order
+    torch.testing.assert_close(dq, want[0], rtol=1e-2, atol=1e-3)
