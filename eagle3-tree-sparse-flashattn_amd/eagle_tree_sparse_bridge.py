@@ -30,6 +30,7 @@ from typing import Callable, Optional, Tuple
 import torch
 
 from tree_sparse_flashattn import (
+    _PLANNED_CALLS,
     BatchedTreeSparseMetadata,
     _check_qkv,
     _layout_ok,
@@ -172,6 +173,7 @@ def run_tree_sparse_kernel(
 # built from the device mask, then the forward, in one C call) per geometry;
 # False marks a geometry that takes the general path.
 _TREE_CALLS: dict = {}
+_PLANNED_CALLS.append(_TREE_CALLS)
 
 
 def _tree_call_plan(q, k, v, mask, block_m, block_n):

@@ -531,12 +531,17 @@ def tree_sparse_attention_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 # launch arguments of forward geometries already validated, by _fwd_key
 _FWD_CALLS: dict = {}
 
+# every table of launch arguments (workspace sizes among them) that a plan
+# under other switches would change; the bridge adds its own
+_PLANNED_CALLS = [_FWD_CALLS]
+
 
 def reload_config() -> None:
     """Re-read the TSFA_* environment switches (the library reads them once)
     and forget launch arguments planned under the old ones."""
     _lib.check("tsfa_config_reload", _lib.load().tsfa_config_reload())
-    _FWD_CALLS.clear()
+    for calls in _PLANNED_CALLS:
+        calls.clear()
 
 
 def _fwd_key(q, k, v, meta, out, return_lse):

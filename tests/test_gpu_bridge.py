@@ -263,3 +263,17 @@ def test_generic_mask_read_matches_the_metadata_route(dtype, b, hq, hkv, t, p, d
         meta = bridge.build_tree_metadata(m, p, 64, 64)
         want = bridge.run_tree_sparse_kernel(q, k, v, None, block_m=64, block_n=64, metadata=meta)
         assert torch.equal(got, want)
+
+
+def test_one_call_path_plans_again_after_a_reload(monkeypatch):
+    # shorter prefix runs need more partials than the remembered workspace holds
+    b, hq, hkv, t, p, d = 1, 8, 2, 24, 1024, 128
+    mask = torch.from_numpy(trees.ancestor_mask(trees.random_parents(t, np.random.default_rng(3)))).cuda()
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)
+               for s in ((b, hq, t, d), (b, hkv, p + t, d), (b, hkv, p + t, d)))
+    monkeypatch.setenv("TSFA_PREFIX_UNITS_PER_SPLIT", "32")
+    want = bridge.run_tree_sparse_kernel(q, k, v, mask, block_m=16, block_n=16)
+    monkeypatch.setenv("TSFA_PREFIX_UNITS_PER_SPLIT", "1")
+    got = bridge.run_tree_sparse_kernel(q, k, v, mask, block_m=16, block_n=16)
+    torch.testing.assert_close(got, want, rtol=1e-2, atol=8e-3)

@@ -142,3 +142,10 @@ def test_paged_rejects_out_shape():
     with pytest.raises(ValueError):
         tsf.tree_sparse_attention_fwd_paged(q, cache, torch.zeros(1, 1, dtype=torch.int32), _cpu_meta(), kv_len=8,
                                             out=torch.zeros(1, 4, 4, 32))
+
+
+def test_reload_config_forgets_every_planned_call():
+    # launch arguments hold workspace sizes of plans made under the old switches
+    tsf._FWD_CALLS["geometry"] = bridge._TREE_CALLS["geometry"] = False
+    tsf.reload_config()
+    assert not tsf._FWD_CALLS and not bridge._TREE_CALLS
