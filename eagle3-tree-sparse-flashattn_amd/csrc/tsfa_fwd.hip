@@ -1725,7 +1725,7 @@ int launch_all(const SplitArgs& sa_in, const CombineArgs& ca, const Plan& p, con
 // v_mfma_f32_32x32x2_f32, with the key order of the P V product permuted so
 // that P^T comes straight from the S^T accumulator.  Every split writes a
 // partial (O / l in the input dtype, fp32 (m, l)) that combine_kernel merges.
-// Units stream HBM -> LDS through a ring of kGenStages(stage bytes) stages
+// Units stream HBM -> LDS through a ring of gen_stages(stage bytes) stages
 // (global_load_lds, NSTG - 1 units ahead).  In the 16-bit instances 16-byte
 // chunk c of key row k sits at chunk position c ^ (k & 15) in the K tile and
 // c ^ ((k & 3) << 2) in the V tile, so the 16 key rows of a K operand read
@@ -1770,22 +1770,8 @@ struct GenArgs {
 // instead of 128 and everything fits the 256 VGPRs, two waves per SIMD
 // (with 128 accumulators, Q and the temporaries the compiler parked O in
 // AGPRs and copied all of it to VGPRs on every unit).  fp32 keeps 4 waves.
-constexpr int kGenRows = 128;
+// (kGenRows, kGenTreeUnits, gen_stages: tsfa_plan.h)
 template <typename T> constexpr int gen_waves() { return sizeof(T) == 2 ? 8 : 4; }
-// Tree units per split whose visibility words the prologue builds into LDS
-// (kGenTreeUnits x 128 rows x 4 bytes after the ring).  Splits with more take
-// the gen_kernel<..., TW = false> instance, which builds each unit's words in
-// the loop: its global loads then make the compiler wait for every vector
-// load in flight (vmcnt(0), which counts the ring's DMA) on every unit, so
-// the ring drains each step.
-constexpr int kGenTreeUnits = 32;
-constexpr size_t kGenTreeBytes = (size_t)kGenTreeUnits * kGenRows * 4;
-// Ring stages for a stage of K+V bytes: as many as fit 128 KB, at least 2,
-// at most 4 (head_dim 256 and fp32 head_dim 128 hold one workgroup per CU by
-// their registers; fp32 head_dim 64 fits two at 64 KB each).
-constexpr int kGenStages(int stage_bytes) {
-  return 131072 / stage_bytes < 2 ? 2 : (131072 / stage_bytes > 4 ? 4 : 131072 / stage_bytes);
-}
 
 constexpr int kGenPre = 1;  // units requested beside Q (at most NSTG - 1)
 
@@ -1798,7 +1784,7 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
   constexpr int CPR = ROWB / 16;            // 16-byte chunks per row
   constexpr int TILE = 32 * ROWB;           // bytes of one unit's K (or V)
   constexpr int SB = 2 * TILE;              // ring stage: K then V
-  constexpr int NSTG = kGenStages(SB);
+  constexpr int NSTG = gen_stages(SB);
   constexpr int LPW = SB / 1024 / NW;  // 1 KB loads per wave per unit
   constexpr int DT = D / 32 / DS;      // O d-tiles of a wave
   constexpr int KS = F32 ? D / 8 : D / 16;  // K reads of S^T: one MFMA each, fp32 four
@@ -2206,65 +2192,6 @@ __global__ __launch_bounds__(gen_waves<T>() * 64) void gen_kernel(const GenArgs 
   }
 }
 
-// The generic kernel's plan: 128-row chunks, the key axis cut into n_slots
-// splits of whole 32-key units: the count with the least modelled time over
-// the rounds of workgroups it makes, with the partials (written once, read
-// once by the combine) held to at most the K/V bytes or 8 MB, whichever is
-// larger (the 8B decode shape at head_dim 256 with fp32 partials: 16 splits,
-// 36.8 us per call, against 40.5 with half the K/V bytes (8 splits, half the
-// CUs idle); twice the K/V bytes: the same 16).
-struct GenPlan {
-  int n_chunks, n_units, units_per_split, n_slots, grid;
-  size_t lds_bytes, ws_acc_bytes, ws_ml_bytes;
-};
-
-inline bool gen_path(int head_dim, int dtype) { return head_dim > 128 || dtype == TSFA_DTYPE_FP32; }
-
-inline int gen_plan(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len, int head_dim, int dtype,
-                    int cus, GenPlan* p) {
-  if (batch <= 0 || q_len <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 || kv_len < 1 || cus <= 0)
-    return TSFA_ERR_INVALID_ARGUMENT;
-  const int64_t TG = (int64_t)q_len * (num_heads / num_kv_heads);
-  if (TG > INT32_MAX / 2) return TSFA_ERR_UNSUPPORTED;
-  p->n_chunks = (int)((TG + kGenRows - 1) / kGenRows);
-  p->n_units = ceil_div(kv_len, 32);
-  const int64_t groups = (int64_t)batch * num_kv_heads * p->n_chunks;
-  const size_t es = dtype == TSFA_DTYPE_FP32 ? 4 : 2;
-  const double kv_bytes = 2.0 * batch * num_kv_heads * (double)kv_len * head_dim * es;
-  const double slot_bytes = (double)batch * num_heads * q_len * ((double)es * head_dim + 8.0);
-  int64_t cap = std::max<int64_t>(1, (int64_t)(std::max(kv_bytes, 8.0 * (1 << 20)) / slot_bytes));
-  // past one workgroup per CU only while the partials fit the allocation-free
-  // forward's array with room to spare
-  const int64_t fill = std::max<int64_t>(1, ((int64_t)cus + groups - 1) / groups);
-  cap = std::min(cap, std::max(fill, (int64_t)(0.75 * TSFA_FWD_NOALLOC_MAX_BYTES / slot_bytes)));
-  // One workgroup per CU, a unit's time and 8 us per workgroup, and with
-  // several splits the combine and the partials at 2 TB/s.  Splits aimed at
-  // one workgroup per CU instead left last rounds nearly empty: 168 groups at
-  // head_dim 256 (3 sequences of 200 tokens behind 3k keys) 2 splits 161 us, 3
-  // 139; 320 fp32 groups (2 of 300 tokens behind 1k keys) 214 -> 201.
-  const double unit_us = dtype == TSFA_DTYPE_FP32 ? 5.0 * head_dim / 128 : 1.9;
-  int slots = 1;
-  double best = 0;
-  for (int want = 1; want <= std::min<int64_t>(std::min(cap, (int64_t)cus), p->n_units); ++want) {
-    const int units = ceil_div(p->n_units, want), n = ceil_div(p->n_units, units);
-    if (n != want) continue;
-    const int64_t rounds = (groups * n + cus - 1) / cus;
-    const double us = (double)rounds * (8.0 + units * unit_us) + (n > 1 ? 5.0 + n * slot_bytes / 2e6 : 0.0);
-    if (want == 1 || us < best) slots = n, best = us;
-  }
-  p->units_per_split = ceil_div(p->n_units, slots);
-  p->n_slots = ceil_div(p->n_units, p->units_per_split);
-  const int64_t grid = groups * p->n_slots;
-  if (grid > INT32_MAX / 2) return TSFA_ERR_UNSUPPORTED;
-  p->grid = (int)grid;
-  const int stage = 2 * 32 * head_dim * (int)es;
-  p->lds_bytes = (size_t)kGenStages(stage) * stage + kGenTreeBytes;
-  const size_t rows = (size_t)batch * num_heads * q_len;
-  p->ws_acc_bytes = align256(rows * p->n_slots * head_dim * es);
-  p->ws_ml_bytes = align256(rows * p->n_slots * 8);
-  return TSFA_OK;
-}
-
 template <typename T, int D, bool TW>
 int launch_gen_kernel(const GenArgs& ga, const GenPlan& p, hipStream_t stream) {
   static std::atomic<uint64_t> attr_set{0};
@@ -2322,36 +2249,61 @@ using namespace tsfa::fwd;
 
 namespace {
 
-// The plan of a shape on the current device (its CU count and LDS limit),
-// memoised per host thread: a call's workspace query and its launch plan the
-// same shape once.
+// The plans this host thread made last, by their keys: a call's workspace
+// query and its launch plan the same shape once.
+template <typename P, int N>
+struct PlanMemo {
+  static constexpr int kEntries = 4;
+  struct Entry {
+    int key[N];
+    P plan;
+    int status;
+  };
+  Entry cache[kEntries] = {};
+  int n_cached = 0, next = 0;
+
+  template <typename Make>
+  int get(const int (&key)[N], P* p, Make make) {
+    for (int e = 0; e < n_cached; ++e)
+      if (std::equal(key, key + N, cache[e].key)) {
+        *p = cache[e].plan;
+        return cache[e].status;
+      }
+    Entry& ent = cache[next];
+    next = (next + 1) % kEntries;
+    n_cached = std::min(n_cached + 1, kEntries);
+    std::copy(key, key + N, ent.key);
+    ent.status = make(&ent.plan);
+    *p = ent.plan;
+    return ent.status;
+  }
+};
+
+// The plan of a shape on the current device (its CU count and LDS limit).
 int device_plan(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len, int prefix_len, int head_dim,
                 bool paged, const Config& cfg, Plan* p) {
   int cus = 0, max_lds = 0;
   if (device_cu_count(&cus) != TSFA_OK || device_max_lds_per_block(&max_lds) != TSFA_OK) return TSFA_ERR_DEVICE;
-  struct Entry {
-    int key[12];
-    Plan plan;
-    int status;
-  };
-  constexpr int kEntries = 4;
-  thread_local Entry cache[kEntries];
-  thread_local int n_cached = 0, next = 0;
-  const int key[12] = {batch, num_heads, num_kv_heads, q_len, kv_len, prefix_len, head_dim, paged ? 1 : 0, cus,
-                       max_lds, cfg.generation, 1};
-  for (int e = 0; e < n_cached; ++e)
-    if (std::equal(key, key + 12, cache[e].key)) {
-      *p = cache[e].plan;
-      return cache[e].status;
-    }
-  Entry& ent = cache[next];
-  next = (next + 1) % kEntries;
-  n_cached = std::min(n_cached + 1, kEntries);
-  std::copy(key, key + 12, ent.key);
-  ent.status = make_plan(batch, num_heads, num_kv_heads, q_len, kv_len, prefix_len, head_dim, paged, cus, max_lds,
-                         cfg, &ent.plan);
-  *p = ent.plan;
-  return ent.status;
+  thread_local PlanMemo<Plan, 11> memo;
+  return memo.get({batch, num_heads, num_kv_heads, q_len, kv_len, prefix_len, head_dim, paged ? 1 : 0, cus, max_lds,
+                   cfg.generation},
+                  p, [&](Plan* out) {
+                    return make_plan(batch, num_heads, num_kv_heads, q_len, kv_len, prefix_len, head_dim, paged, cus,
+                                     max_lds, cfg, out);
+                  });
+}
+
+// The same for the generic kernel (no switch changes its plan): searched anew
+// at a call's two queries, its split counts took 0.1 us (one unit) to 0.7 us
+// (256 and 512 units) of host time per call.
+int device_gen_plan(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len, int head_dim, int dtype,
+                    GenPlan* p) {
+  int cus = 0;
+  if (device_cu_count(&cus) != TSFA_OK) return TSFA_ERR_DEVICE;
+  thread_local PlanMemo<GenPlan, 8> memo;
+  return memo.get({batch, num_heads, num_kv_heads, q_len, kv_len, head_dim, dtype, cus}, p, [&](GenPlan* out) {
+    return make_gen_plan(batch, num_heads, num_kv_heads, q_len, kv_len, head_dim, dtype, cus, out);
+  });
 }
 
 }  // namespace
@@ -2360,11 +2312,8 @@ extern "C" size_t tsfa_fwd_workspace_bytes_for_dtype(int batch, int num_heads, i
                                                      int kv_len, int prefix_len, int head_dim, int dtype) {
   if (batch <= 0 || q_len <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0) return 0;
   if (gen_path(head_dim, dtype)) {
-    int cus = 0;
     GenPlan gp;
-    if (device_cu_count(&cus) != TSFA_OK ||
-        gen_plan(batch, num_heads, num_kv_heads, q_len, kv_len, head_dim, dtype, cus, &gp) != TSFA_OK)
-      return 0;
+    if (device_gen_plan(batch, num_heads, num_kv_heads, q_len, kv_len, head_dim, dtype, &gp) != TSFA_OK) return 0;
     return gp.ws_acc_bytes + gp.ws_ml_bytes;
   }
   // enough for both the contiguous and the paged plan of the shape
@@ -2452,10 +2401,8 @@ int gen_impl(const void* q, const KvSource& kv, void* o, float* lse, const TreeS
              int kv_len, int prefix_len, int gqa_group_size, int block_m, int block_n, int head_dim, int dtype,
              void* workspace, size_t workspace_bytes, hipStream_t stream, const int64_t* q_strides) {
   if (kv.paged()) return TSFA_ERR_UNSUPPORTED;
-  int cus = 0;
-  if (device_cu_count(&cus) != TSFA_OK) return TSFA_ERR_DEVICE;
   GenPlan p;
-  int st = gen_plan(batch, num_heads, num_kv_heads, q_len, kv_len, head_dim, dtype, cus, &p);
+  int st = device_gen_plan(batch, num_heads, num_kv_heads, q_len, kv_len, head_dim, dtype, &p);
   if (st != TSFA_OK) return st;
   if (workspace == nullptr || workspace_bytes < p.ws_acc_bytes + p.ws_ml_bytes ||
       reinterpret_cast<uintptr_t>(workspace) % 256 != 0)

@@ -208,6 +208,61 @@ size_t workspace_bytes(int batch, int num_heads, int num_kv_heads, int q_len, in
   return std::max(p.ws_acc_bytes + p.ws_ml_bytes, pp.ws_acc_bytes + pp.ws_ml_bytes);
 }
 
+// The generic kernel's plan: 128-row chunks, the key axis cut into n_slots
+// splits of whole 32-key units: the count with the least modelled time over
+// the rounds of workgroups it makes, with the partials (written once, read
+// once by the combine) held to at most the K/V bytes or 8 MB, whichever is
+// larger (the 8B decode shape at head_dim 256 with fp32 partials: 16 splits,
+// 36.8 us per call, against 40.5 with half the K/V bytes (8 splits, half the
+// CUs idle); twice the K/V bytes: the same 16).
+int make_gen_plan(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len, int head_dim, int dtype, int cus,
+                  GenPlan* p) {
+  if (batch <= 0 || q_len <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 || kv_len < 1 || cus <= 0)
+    return TSFA_ERR_INVALID_ARGUMENT;
+  const int64_t TG = (int64_t)q_len * (num_heads / num_kv_heads);
+  if (TG > INT32_MAX / 2) return TSFA_ERR_UNSUPPORTED;
+  p->n_chunks = (int)((TG + kGenRows - 1) / kGenRows);
+  p->n_units = ceil_div(kv_len, 32);
+  const int64_t groups = (int64_t)batch * num_kv_heads * p->n_chunks;
+  const size_t es = dtype == TSFA_DTYPE_FP32 ? 4 : 2;
+  const double kv_bytes = 2.0 * batch * num_kv_heads * (double)kv_len * head_dim * es;
+  const double slot_bytes = (double)batch * num_heads * q_len * ((double)es * head_dim + 8.0);
+  int64_t cap = std::max<int64_t>(1, (int64_t)(std::max(kv_bytes, 8.0 * (1 << 20)) / slot_bytes));
+  // past one workgroup per CU only while the partials fit the allocation-free
+  // forward's array with room to spare
+  const int64_t fill = std::max<int64_t>(1, ((int64_t)cus + groups - 1) / groups);
+  cap = std::min(cap, std::max(fill, (int64_t)(0.75 * TSFA_FWD_NOALLOC_MAX_BYTES / slot_bytes)));
+  // One workgroup per CU, a unit's time and 8 us per workgroup, and with
+  // several splits the combine and the partials at 2 TB/s.  Splits aimed at
+  // one workgroup per CU instead left last rounds nearly empty: 168 groups at
+  // head_dim 256 (3 sequences of 200 tokens behind 3k keys) 2 splits 161 us, 3
+  // 139; 320 fp32 groups (2 of 300 tokens behind 1k keys) 214 -> 201.  Two
+  // fp32 workgroups of head_dim 64 fit a CU and share its matrix rate: counted
+  // as two places (a unit 2.5, 4 or 5 us) 24 drawn shapes of 60 to 700 groups
+  // ran 0.83 to 1.21 times as fast as counted as one, 0.99 to 1.00 on average.
+  const double unit_us = dtype == TSFA_DTYPE_FP32 ? 5.0 * head_dim / 128 : 1.9;
+  int slots = 1;
+  double best = 0;
+  for (int want = 1; want <= std::min<int64_t>(std::min(cap, (int64_t)cus), p->n_units); ++want) {
+    const int units = ceil_div(p->n_units, want), n = ceil_div(p->n_units, units);
+    if (n != want) continue;
+    const int64_t rounds = (groups * n + cus - 1) / cus;
+    const double us = (double)rounds * (8.0 + units * unit_us) + (n > 1 ? 5.0 + n * slot_bytes / 2e6 : 0.0);
+    if (want == 1 || us < best) slots = n, best = us;
+  }
+  p->units_per_split = ceil_div(p->n_units, slots);
+  p->n_slots = ceil_div(p->n_units, p->units_per_split);
+  const int64_t grid = groups * p->n_slots;
+  if (grid > INT32_MAX / 2) return TSFA_ERR_UNSUPPORTED;
+  p->grid = (int)grid;
+  const int stage = 2 * 32 * head_dim * (int)es;
+  p->lds_bytes = (size_t)gen_stages(stage) * stage + kGenTreeBytes;
+  const size_t rows = (size_t)batch * num_heads * q_len;
+  p->ws_acc_bytes = align256(rows * p->n_slots * head_dim * es);
+  p->ws_ml_bytes = align256(rows * p->n_slots * 8);
+  return TSFA_OK;
+}
+
 int check_args(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len, int prefix_len, int n_q_blocks,
                int n_tree_blocks, int gqa_group_size, int block_m, int block_n, int head_dim, int dtype) {
   if (batch < 0 || num_heads <= 0 || num_kv_heads <= 0 || q_len < 0) return TSFA_ERR_INVALID_ARGUMENT;

@@ -98,6 +98,33 @@ int make_plan(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len,
 size_t workspace_bytes(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len, int prefix_len,
                        int head_dim, int cus, int max_lds);
 
+// Generic kernel (head_dim 256, fp32): rows of a chunk.
+constexpr int kGenRows = 128;
+// Tree units per split whose visibility words the prologue builds into LDS
+// (kGenTreeUnits x 128 rows x 4 bytes after the ring).  Splits with more take
+// the gen_kernel<..., TW = false> instance, which builds each unit's words in
+// the loop: its global loads then make the compiler wait for every vector
+// load in flight (vmcnt(0), which counts the ring's DMA) on every unit, so
+// the ring drains each step.
+constexpr int kGenTreeUnits = 32;
+constexpr size_t kGenTreeBytes = (size_t)kGenTreeUnits * kGenRows * 4;
+// Ring stages for a stage of K+V bytes: as many as fit 128 KB, at least 2,
+// at most 4 (head_dim 256 and fp32 head_dim 128 hold one workgroup per CU by
+// their registers and LDS; of fp32 head_dim 64, 80 KB with the words, two fit).
+constexpr int gen_stages(int stage_bytes) {
+  return 131072 / stage_bytes < 2 ? 2 : (131072 / stage_bytes > 4 ? 4 : 131072 / stage_bytes);
+}
+
+inline bool gen_path(int head_dim, int dtype) { return head_dim > 128 || dtype == TSFA_DTYPE_FP32; }
+
+struct GenPlan {
+  int n_chunks, n_units, units_per_split, n_slots, grid;
+  size_t lds_bytes, ws_acc_bytes, ws_ml_bytes;
+};
+
+int make_gen_plan(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len, int head_dim, int dtype, int cus,
+                  GenPlan* p);
+
 int check_args(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len, int prefix_len, int n_q_blocks,
                int n_tree_blocks, int gqa_group_size, int block_m, int block_n, int head_dim, int dtype);
 

@@ -11,6 +11,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <random>
 #include <vector>
 
@@ -119,6 +120,46 @@ static void sweep_fwd_plan() {
   EXPECT(fwd::make_plan(1, 4, 2, 8, 8, 0, 128, false, 256, 1024, c0, &p) == TSFA_ERR_UNSUPPORTED, "small LDS");
   EXPECT(fwd::make_plan(1, 4096, 1, (1 << 30), (1 << 30), 0, 128, false, 256, 163840, c0, &p) ==
              TSFA_ERR_UNSUPPORTED, "huge rows");
+}
+
+// The generic kernel's splits: whole units, none empty, within the LDS; and no
+// more partials than the allocation-free forward's array where one split per
+// idle compute unit fits it.
+static void sweep_gen_plan() {
+  const int cus_list[] = {1, 8, 80, 256, 304};
+  for (int it = 0; it < 60000; ++it) {
+    const int kvh = (int)uni(1, 16), g = (int)uni(1, 16), batch = (int)uni(1, 64), heads = kvh * g;
+    const int q_len = (int)uni(1, it % 10 == 0 ? 20000 : 1100);
+    const int kv_len = q_len + (int)uni(0, it % 7 == 0 ? 300000 : 20000), cus = cus_list[uni(0, 4)];
+    const int dtype = uni(0, 1) ? TSFA_DTYPE_FP32 : TSFA_DTYPE_BF16;
+    const int D = dtype == TSFA_DTYPE_FP32 ? 64 << uni(0, 2) : 256, es = dtype == TSFA_DTYPE_FP32 ? 4 : 2;
+    fwd::GenPlan p;
+    memset(&p, 0xAB, sizeof(p));
+    const int st = fwd::make_gen_plan(batch, heads, kvh, q_len, kv_len, D, dtype, cus, &p);
+    EXPECT(st == TSFA_OK, "status %d", st);
+    if (st != TSFA_OK) continue;
+    const int64_t TG = (int64_t)q_len * g;
+    EXPECT((int64_t)p.n_chunks * fwd::kGenRows >= TG && (int64_t)(p.n_chunks - 1) * fwd::kGenRows < TG, "chunks");
+    EXPECT(p.n_units == (kv_len + 31) / 32 && p.units_per_split >= 1 && p.n_slots >= 1, "units");
+    EXPECT((int64_t)p.n_slots * p.units_per_split >= p.n_units &&
+               (int64_t)(p.n_slots - 1) * p.units_per_split < p.n_units,
+           "slots %d of %d units, %d in all", p.n_slots, p.units_per_split, p.n_units);
+    const int64_t groups = (int64_t)batch * kvh * p.n_chunks;
+    EXPECT(p.grid == groups * p.n_slots, "grid");
+    const int stage = 2 * 32 * D * es, stages = fwd::gen_stages(stage);
+    EXPECT(stages >= 2 && p.lds_bytes == (size_t)stages * stage + fwd::kGenTreeBytes && p.lds_bytes <= 163840, "lds");
+    const size_t rows = (size_t)batch * heads * q_len;
+    EXPECT(p.ws_acc_bytes >= rows * p.n_slots * D * es && p.ws_ml_bytes >= rows * p.n_slots * 8, "workspace");
+    const int64_t fill = std::max<int64_t>(1, (cus + groups - 1) / groups);
+    const size_t limit = TSFA_FWD_NOALLOC_MAX_BYTES;
+    if (rows * std::min<int64_t>(fill, p.n_units) * (D * es + 8) + 512 <= limit)
+      EXPECT(p.ws_acc_bytes + p.ws_ml_bytes <= limit, "%zu bytes of partials", p.ws_acc_bytes + p.ws_ml_bytes);
+  }
+  fwd::GenPlan p;
+  EXPECT(fwd::make_gen_plan(0, 4, 2, 8, 8, 256, TSFA_DTYPE_BF16, 256, &p) != TSFA_OK, "batch 0");
+  EXPECT(fwd::make_gen_plan(1, 5, 2, 8, 8, 256, TSFA_DTYPE_BF16, 256, &p) != TSFA_OK, "heads");
+  EXPECT(fwd::make_gen_plan(1, 4, 2, 8, 0, 256, TSFA_DTYPE_BF16, 256, &p) != TSFA_OK, "no keys");
+  EXPECT(fwd::make_gen_plan(1, 4, 2, 8, 8, 256, TSFA_DTYPE_BF16, 0, &p) != TSFA_OK, "no CUs");
 }
 
 static void sweep_check_args() {
@@ -296,6 +337,7 @@ static void sweep_meta() {
 int main() {
   sweep_fastdiv();
   sweep_fwd_plan();
+  sweep_gen_plan();
   sweep_check_args();
   sweep_layouts();
   sweep_bwd_plan();
