@@ -47,16 +47,15 @@ constexpr int kPlaceGroups = 512;  // workgroups per sequence of the place kerne
 // Bits [32*wi, 32*wi + 32) of block (qb, tb) of the sequence whose mask
 // starts at m0, zero-padded past the block's clipped h x w extent (:44-64).
 // (r0, c0): row and column of the word's first bit, flat = 32 * wi.
-// When the 32 bits lie in one block row the word is two 16-byte loads, at
-// any alignment (the device takes unaligned vector loads; the masks of odd
-// tree lengths have odd row strides): a row's last word, cut by the mask's
-// edge, comes from the 32 bytes that end at the edge, shifted down, when the
-// mask row reaches that far back.  Byte loads are left for words that wrap
-// block rows and masks under 32 columns; all are issued before any is used
-// (addresses clamped to the block's first byte where the bit is padding), so
-// a word costs one memory latency -- but 32 load instructions per wave: a
-// 61-token tree in one 64 x 64 block took 8.4 us that way, 2.5 us with
-// vector loads.
+// When the 32 bits lie in one block row they are a word of the mask's row
+// (mask_word: two 16-byte loads at any alignment -- the masks of odd tree
+// lengths have odd row strides -- and rows of under 32 columns 8 bytes at a
+// time).  Byte loads are left for words that wrap block rows; all are issued
+// before any is used (addresses clamped to the block's first byte where the
+// bit is padding), so a word costs one memory latency -- but 32 load
+// instructions per wave: a 61-token tree in one 64 x 64 block took 8.4 us
+// that way, 2.5 us with vector loads, trees of 5 to 31 tokens 7.5-7.7 us and
+// 2.3-2.9.
 __device__ inline uint32_t block_word_at(const uint8_t* m0, int64_t row_stride, const MetaGeom& g, int qb, int tb,
                                          int64_t flat, int r0, int c0) {
   const int q0 = qb * g.block_m, k0 = tb * g.block_n;
@@ -65,9 +64,8 @@ __device__ inline uint32_t block_word_at(const uint8_t* m0, int64_t row_stride, 
   const uint8_t* m = m0 + (int64_t)q0 * row_stride + k0;
   const int64_t n_flat = (int64_t)g.block_m * g.block_n;
   if (c0 + 32 <= g.block_n) {
-    const int valid = min(32, w - c0);  // bits inside the clipped block
-    if (r0 >= h || valid <= 0) return 0;
-    if (k0 + c0 + valid >= 32) return pack32(m + (int64_t)r0 * row_stride + c0 + valid - 32) >> (32 - valid);
+    if (r0 >= h || c0 >= w) return 0;
+    return mask_word(m0 + (int64_t)(q0 + r0) * row_stride, k0 + c0, g.q_len);
   }
   uint8_t v[32];
   bool in[32];

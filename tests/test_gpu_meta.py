@@ -118,3 +118,18 @@ def test_pack_block(shape):
     m[-1, -1] = True
     got = tsf._pack_block_mask_to_int32(torch.from_numpy(m).cuda())
     np.testing.assert_array_equal(got.cpu().numpy(), mo.pack_block_bits(m))
+
+
+# rows of under 32 columns inside wider blocks (words cut by the mask's edge
+# and not reaching back 32 columns), at unaligned bases and strides
+@pytest.mark.parametrize("path", ["auto", "two-launch"])
+@pytest.mark.parametrize("q_len,bm,bn", [(1, 16, 64), (5, 64, 64), (7, 4, 32), (8, 64, 48), (20, 16, 128), (31, 1, 40)])
+def test_short_rows(q_len, bm, bn, path, monkeypatch):
+    if path == "two-launch":
+        monkeypatch.setenv("TSFA_META_SMALL", "0")
+    rng = np.random.default_rng(q_len)
+    wide = torch.from_numpy(rng.random((3, q_len, q_len + 5)) < 0.4).cuda()
+    masks = wide[:, :, 3:3 + q_len]
+    got = tsf.prepare_tree_sparse_metadata_batched(masks, 11, bm, bn)
+    for b in range(3):
+        assert_meta_equal(got.sequence(b), mo.build_metadata(masks[b].cpu().numpy(), 11, bm, bn))
