@@ -1189,7 +1189,6 @@ void split_kernel(const SplitArgs a) {
     const int tok_hi = (int)fdiv(row0 + rows_chunk - 1, a.fd_group);  // tokens tok_lo .. tok_hi
     const int ntok = tok_hi - tok_lo + 1;
     const int qb_lo = tok_lo / BM, qb_hi = tok_hi / BM, nqbc = qb_hi - qb_lo + 1;
-    const int n_tu = (a.tree_key_limit + kUnitKeys - 1) / kUnitKeys;
     const int32_t* rp = a.row_ptr + b * a.ms_row_ptr;
     const int32_t* ci = a.col_idx + b * a.ms_col_idx;
     const int8_t* bt = a.blk_type + b * a.ms_blk_type;
@@ -1215,6 +1214,7 @@ void split_kernel(const SplitArgs a) {
     auto build_state = [&]() {
       for (int i = tid; i < n_st; i += kWaves * 64) st[i] = 0;
       if constexpr (MASK) {
+        const int n_tu = (a.tree_key_limit + kUnitKeys - 1) / kUnitKeys;
         sync_lds();
         for (int i = tid; i < w_rows * n_tu; i += kWaves * 64) {
           const int row = i / n_tu, u = i - row * n_tu;
@@ -1241,6 +1241,7 @@ void split_kernel(const SplitArgs a) {
     build_state();
     TSFA_STAMP(44);
     // Tree units holding a key some row of the chunk can see, compacted.
+    const int n_tu = (a.tree_key_limit + kUnitKeys - 1) / kUnitKeys;
     for (int i = tid; i < n_tu; i += kWaves * 64) vis[i] = 0;
     sync_lds();
     for (int i = tid; i < n_st; i += kWaves * 64) {
@@ -1649,8 +1650,7 @@ int launch_all(const SplitArgs& sa_in, const CombineArgs& ca, const Plan& p, con
                                : fm == 1 ? (ptab ? launch_split<T, D, 1, true, false, D == 128 ? 9 : 1>(sa, pt, stream)
                                                  : launch_split<T, D, 1, true, false, 1>(sa, p, stream))
                                          : launch_split<T, D, 1, true, false>(sa, p, stream));
-    else
-    {
+    else {
       auto go = [&](auto s_c, auto f_c) {
         constexpr int S = decltype(s_c)::value, F = decltype(f_c)::value;
         return sa.mask != nullptr ? launch_split<T, D, S, false, false, F | 16>(sa, p, stream)
