@@ -59,6 +59,7 @@ namespace bwd {
 
 constexpr int kWaves = 8;                 // 4 key groups x 2 row groups
 // kBlockKeys, kTileRows, kMaxStateInts: tsfa_plan.h
+static_assert(kWaves * 64 == kMainThreads, "launch size");
 constexpr int kBufs = 2;                  // Q / dO tile buffers per row group: loads run one step ahead
 
 // 16-byte-chunk XOR swizzle of a row-major [rows][D] LDS tile (row period
@@ -1027,10 +1028,12 @@ int launch_bwd(const BwdArgs& ba, const PrepArgs& pa, const VisArgs& va, const D
                          stream, a);
     return hipGetLastError() == hipSuccess;
   };
-  // TSFA_BWD_CONCURRENT=0: one pass after the other (measurements)
+  // TSFA_BWD_CONCURRENT=0 (measurements), or more threads than a grid holds:
+  // one pass after the other
   const int n1 = 8 * (ba.dq_first ? ba.q_pairs_per_xcd : ba.items_per_xcd);
   const int n2 = 8 * (ba.dq_first ? ba.items_per_xcd : ba.q_pairs_per_xcd);
-  if (config().bwd_concurrent != 0 ? !launch_main(0, n1 + n2) : !launch_main(0, n1) || !launch_main(n1, n2))
+  const bool joint = config().bwd_concurrent != 0 && one_launch(n1, n2);
+  if (joint ? !launch_main(0, n1 + n2) : !launch_main(0, n1) || !launch_main(n1, n2))
     return TSFA_ERR_LAUNCH;
   if (ba.dq_direct) return TSFA_OK;
   const int64_t dq_threads = (int64_t)da.batch * da.num_kv_heads * da.q_len * da.group * (D / 8);

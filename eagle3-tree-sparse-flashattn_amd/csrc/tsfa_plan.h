@@ -166,6 +166,11 @@ int make_bwd_plan(int batch, int num_kv_heads, int q_len, int kv_len, int prefix
 bool tile_offsets_fit(int gqa, int64_t sh, int64_t sm, int head_dim);
 bool unit_offsets_fit(int64_t sn, int head_dim);
 
+constexpr int kMainThreads = 512;  // threads of a workgroup of the main launch
+// Whether the two passes' workgroups fit one launch: a grid holds at most
+// 2^32 - 1 threads.
+inline bool one_launch(int64_t n1, int64_t n2) { return n1 + n2 <= (int64_t)UINT32_MAX / kMainThreads; }
+
 constexpr int kMaxDqSplits = 16;
 
 // Key splits of each of the dQ pass's `chunks` 128-row chunks (all groups

@@ -233,6 +233,26 @@ static void sweep_bwd_plan() {
   }
 }
 
+// The dQ pass's key splits: whole 32-key units, none empty, at most
+// kMaxDqSplits; and no joint launch of more threads than a grid holds.
+static void sweep_dq_splits() {
+  const int cus_list[] = {1, 8, 80, 256, 304};
+  for (int it = 0; it < 40000; ++it) {
+    const int64_t kv_items = uni(0, it % 9 == 0 ? 2000000 : 5000), chunks = uni(1, it % 11 == 0 ? 500000 : 3000);
+    const int steps = (int)uni(1, it % 7 == 0 ? 60000 : 300), n_units = (int)uni(1, it % 5 == 0 ? 70000 : 1200);
+    int splits = -1;
+    bool first = false;
+    bwd::dq_split_plan(kv_items, steps, chunks, n_units, uni(0, 1) ? 64 : 128, uni(0, 1ll << 36), cus_list[uni(0, 4)],
+                       &splits, &first);
+    EXPECT(splits >= 1 && splits <= std::min(bwd::kMaxDqSplits, n_units), "%d splits of %d units", splits, n_units);
+    const int units = ceil_div(n_units, std::max(1, splits));
+    EXPECT(ceil_div(n_units, units) == splits, "%d splits of %d units leave one empty", splits, n_units);
+  }
+  EXPECT(bwd::one_launch(264, 32) && bwd::one_launch(8388000, 0) && !bwd::one_launch(5600000, 2800000) &&
+             !bwd::one_launch(INT32_MAX / 2, INT32_MAX / 2),
+         "launch size");
+}
+
 // The backward's scalar-base loads: where the rule allows them, every lane
 // offset of a tile (unit), formed in 64 bits, is what 32 unsigned bits hold.
 static void sweep_bwd_offsets() {
@@ -342,6 +362,7 @@ int main() {
   sweep_layouts();
   sweep_bwd_plan();
   sweep_bwd_offsets();
+  sweep_dq_splits();
   sweep_meta();
   if (g_fail) {
     fprintf(stderr, "%d invariant violations\n", g_fail);
