@@ -248,6 +248,22 @@ static void sweep_dq_splits() {
     const int units = ceil_div(n_units, std::max(1, splits));
     EXPECT(ceil_div(n_units, units) == splits, "%d splits of %d units leave one empty", splits, n_units);
   }
+  // the shapes of tests/test_gpu_bwd.py that stand for dQ workgroups first, on
+  // 256 compute units (batch, kv heads, group, tokens, prefix, head_dim, splits)
+  const int shapes[][7] = {{15, 9, 2, 45, 100, 128, 1}, {3, 29, 7, 20, 130, 64, 1}, {5, 17, 2, 45, 200, 64, 1},
+                           {9, 7, 2, 16, 500, 128, 3}, {2, 16, 7, 16, 1000, 64, 3}};
+  for (const auto& s : shapes) {
+    bwd::BwdPlan p;
+    EXPECT(bwd::make_bwd_plan(s[0], s[1], s[3], s[4] + s[3], s[4], s[2], s[5], 16, ceil_div(s[3], 16), 1, &p) == TSFA_OK,
+           "plan");
+    const int64_t bk = (int64_t)s[0] * s[1];
+    int splits = 0;
+    bool first = false;
+    bwd::dq_split_plan(bk * (p.n_pb + p.n_tb), (p.n_tiles + 1) / 2, bk * ceil_div(p.n_tiles, 4),
+                       ceil_div(s[4], 32) + ceil_div(s[3], 32), s[5], (int64_t)p.dq_bytes, 256, &splits, &first);
+    EXPECT(first && splits == s[6], "%d tokens of %lld heads: %d splits, dQ first %d", s[3], (long long)bk, splits,
+           (int)first);
+  }
   EXPECT(bwd::one_launch(264, 32) && bwd::one_launch(8388000, 0) && !bwd::one_launch(5600000, 2800000) &&
              !bwd::one_launch(INT32_MAX / 2, INT32_MAX / 2),
          "launch size");

@@ -61,9 +61,9 @@ def _check(name, got, ref, dtype):
     assert err <= bound, f"{name}: max_abs_err {err:.3e} > {bound:.3e}"
 
 
-def _run_and_check(q, k, v, do, mask, p, bm, bn, dtype, sm_scale=None, batched=False):
+def _run_and_check(q, k, v, do, mask, p, bm, bn, dtype, sm_scale=None, batched=False, layout=None):
     dev = torch.device("cuda", 0)
-    qd, kd, vd, dod = (x.to(dev) for x in (q, k, v, do))
+    qd, kd, vd, dod = (x.to(dev) if layout is None else layout(x.to(dev)) for x in (q, k, v, do))
     if batched:
         meta = tsf.prepare_tree_sparse_metadata_batched(mask.to(dev), p, bm, bn)
     else:
@@ -284,3 +284,56 @@ def test_bwd_reversed_rows_and_keys():
     assert torch.equal(dk, want[1]) and torch.equal(dv, want[2])
     # dQ sums fp32 atomics of the key splits in a run-dependent order
     torch.testing.assert_close(dq, want[0], rtol=1e-2, atol=1e-3)
+
+
+# Shapes whose dQ workgroups the planner puts before the dK / dV ones on 256
+# compute units (tests/sanitize/plan_sweep.cpp checks that it does): dQ written
+# directly or split, odd counts of items, so that the last workgroup has one
+# half, odd counts of units, groups that do not divide 32
+DQ_FIRST = [
+    # b, hq, hkv, t, p, d, dtype: key splits, items
+    (15, 18, 9, 45, 100, 128, BF),     # 1, 135
+    (3, 203, 29, 20, 130, 64, FP),     # 1, 174 (7 query heads per kv head)
+    (5, 34, 17, 45, 200, 64, BF),      # 1, 85
+    (9, 14, 7, 16, 500, 128, FP),      # 3, 189
+    (2, 112, 16, 16, 1000, 64, BF),    # 3, 96 (7 query heads per kv head)
+]
+
+
+@pytest.mark.parametrize("case", DQ_FIRST, ids=[f"f{i}" for i in range(len(DQ_FIRST))])
+def test_bwd_dq_workgroups_first(case, monkeypatch):
+    b, hq, hkv, t, p, d, dtype = case
+    print(f"[bwd] dQ first {case}", flush=True)
+    mask = torch.from_numpy(_tree("random", t, np.random.default_rng(t)))
+    ins = _inputs(b, hq, hkv, t, p, d, dtype, seed=t + p)
+    dq, dk, dv = _run_and_check(*ins, mask, p, 16, 16, dtype)
+    # the same two passes, one launch each
+    monkeypatch.setenv("TSFA_BWD_CONCURRENT", "0")
+    dq2, dk2, dv2 = _run_and_check(*ins, mask, p, 16, 16, dtype)
+    assert torch.equal(dk, dk2) and torch.equal(dv, dv2)
+    if case in DQ_FIRST[:3]:  # (split, dQ sums fp32 atomics in a run-dependent order)
+        assert torch.equal(dq, dq2)
+
+
+def _transposed(x):  # a [B, N, H, D] projection seen as [B, H, N, D]
+    return x.transpose(1, 2).contiguous().transpose(1, 2)
+
+
+def _sliced(x):  # a slice of a wider fused projection, [B, N, 3, H, D + 8]
+    b, h, n, d = x.shape
+    wide = torch.full((b, n, 3, h, d + 8), float("nan"), dtype=x.dtype, device=x.device)
+    wide[:, :, 1, :, :d] = x.transpose(1, 2)
+    return wide[:, :, 1, :, :d].transpose(1, 2)
+
+
+# q, k, v and dO (and, where their layout is dense, the gradients) off the
+# dense [B, H, N, D] layout: the scalar-base loads of whole tiles and units,
+# and the general ones of a group that does not divide 32, over several units
+# per split and tiles past the end
+@pytest.mark.parametrize("layout", [_transposed, _sliced])
+@pytest.mark.parametrize("b,hq,hkv,t,p,d,dtype", [(2, 8, 2, 96, 600, 64, FP), (1, 32, 8, 64, 1000, 128, BF),
+                                                  (1, 28, 4, 150, 800, 128, BF), (2, 14, 2, 37, 333, 64, FP)])
+def test_bwd_strided_inputs(b, hq, hkv, t, p, d, dtype, layout):
+    print(f"[bwd] {layout.__name__} b={b} hq={hq} hkv={hkv} t={t} p={p} d={d}", flush=True)
+    mask = torch.from_numpy(_tree("eagle" if t < 100 else "random", t, np.random.default_rng(t)))
+    _run_and_check(*_inputs(b, hq, hkv, t, p, d, dtype, seed=t), mask, p, 16, 32, dtype, layout=layout)
