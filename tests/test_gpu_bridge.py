@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from oracle import meta_oracle
-from tsfa import trees
+from tsfa import _lib, trees
 from tests.gpu_util import assert_close_to_oracle, oracle_out
 
 pytestmark = pytest.mark.gpu
@@ -213,18 +213,40 @@ def test_one_call_path_refuses_kv_shorter_than_q():
                                       block_m=16, block_n=32)
 
 
+def _tree_call_route(q, k, v, mask, bm, bn):
+    """Which kernels tsfa_tree_attention read the mask with: the metadata
+    builder writes its record's row_ptr, [0] = 0 first, at the front of the
+    workspace; the attention kernels' own mask read leaves it alone."""
+    strides, ints, ws_bytes, scale, n_masks, seq_stride, row_stride = bridge._tree_call_plan(q, k, v, mask, bm, bn)
+    ws = torch.full((ws_bytes,), 0xA5, dtype=torch.uint8, device="cuda")
+    out = torch.empty_like(q)
+    lib = _lib.load()
+    st = lib.tsfa_tree_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mask.data_ptr(), seq_stride,
+                                 row_stride, n_masks, strides, scale, *ints, ws.data_ptr(), ws_bytes,
+                                 _lib.stream_handle(q.device))
+    _lib.check("tsfa_tree_attention", st)
+    return "builder" if ws[:4].cpu().tolist() == [0] * 4 else "mask"
+
+
 # the split kernel's own mask read (tiles of 32 columns, cut and short rows,
 # q-blocks wider than a chunk, several word batches per chunk, one and two key
-# streams, one-slot plans, trees without a prefix) against the metadata route:
-# the same units in the same order, so the same bits
-@pytest.mark.parametrize("b,hq,hkv,t,p,d,bm,bn", [
-    (1, 4, 4, 1, 64, 64, 64, 64), (1, 4, 2, 7, 96, 128, 16, 16), (2, 8, 8, 31, 33, 64, 64, 48),
-    (2, 4, 2, 3, 96, 64, 16, 16), (1, 4, 4, 2, 64, 128, 16, 16), (1, 8, 2, 13, 96, 64, 16, 32), (1, 8, 2, 16, 64, 128, 16, 16),
-    (3, 14, 2, 33, 1024, 64, 64, 64), (1, 32, 8, 61, 4095, 128, 16, 32), (16, 8, 2, 64, 2048, 128, 16, 64),
-    (1, 8, 1, 200, 500, 128, 128, 128), (2, 4, 1, 95, 0, 128, 32, 64), (1, 4, 2, 1100, 640, 64, 16, 64),
-    (1, 2, 2, 1200, 320, 128, 64, 64), (1, 8, 1, 515, 2048, 128, 1, 16)])
-def test_mask_read_in_the_kernel_matches_the_metadata_route(b, hq, hkv, t, p, d, bm, bn):
-    print(f"[bridge] mask read b={b} hq={hq} hkv={hkv} t={t} p={p} d={d} bm={bm} bn={bn}", flush=True)
+# streams, one-slot plans, trees without a prefix, windows of mask rows up to
+# the limit) against the metadata route: the same units in the same order, so
+# the same bits; and the calls that keep the builder (windows past the limit,
+# the checked ring steps)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,hq,hkv,t,p,d,bm,bn,route", [
+    (1, 4, 4, 1, 64, 64, 64, 64, "mask"), (1, 4, 2, 7, 96, 128, 16, 16, "mask"), (2, 8, 8, 31, 33, 64, 64, 48, "mask"),
+    (2, 4, 2, 3, 96, 64, 16, 16, "mask"), (1, 4, 4, 2, 64, 128, 16, 16, "mask"), (1, 8, 2, 13, 96, 64, 16, 32, "mask"),
+    (1, 8, 2, 16, 64, 128, 16, 16, "mask"), (3, 14, 2, 33, 1024, 64, 64, 64, "mask"),
+    (1, 32, 8, 61, 4095, 128, 16, 32, "mask"), (16, 8, 2, 64, 2048, 128, 16, 64, "mask"),
+    (1, 8, 1, 200, 500, 128, 128, 128, "mask"), (2, 4, 1, 95, 0, 128, 32, 64, "mask"),
+    (1, 4, 2, 1100, 640, 64, 16, 64, "mask"), (1, 8, 1, 515, 2048, 128, 1, 16, "mask"),
+    # 130 rows of 2016 (2017) bytes: 262080 (262210), the limit 262144
+    (1, 4, 2, 2016, 64, 64, 1, 16, "mask"), (1, 4, 2, 2017, 64, 64, 1, 16, "builder"),
+    (1, 2, 2, 1200, 320, 128, 64, 64, "builder"), (2, 4, 2, 3, 97, 64, 16, 16, "builder")])
+def test_mask_read_in_the_kernel_matches_the_metadata_route(b, hq, hkv, t, p, d, bm, bn, route, dtype):
+    print(f"[bridge] mask read b={b} hq={hq} hkv={hkv} t={t} p={p} d={d} bm={bm} bn={bn} {dtype}", flush=True)
     rng = np.random.default_rng(t)
     masks = np.stack([trees.ancestor_mask(trees.depth_limited_parents(t, 6, rng)) for _ in range(b)])
     masks[0, t // 2] = False  # a row that sees no tree key
@@ -233,10 +255,13 @@ def test_mask_read_in_the_kernel_matches_the_metadata_route(b, hq, hkv, t, p, d,
     wide[:, :, 1:1 + t] = torch.from_numpy(masks).cuda()
     mask = wide[:, :, 1:1 + t]  # unaligned rows
     g = torch.Generator(device="cuda").manual_seed(t)
-    q, k, v = (torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)
+    q, k, v = (torch.randn(s, generator=g, device="cuda").to(dtype)
                for s in ((b, hq, t, d), (b, hkv, p + t, d), (b, hkv, p + t, d)))
     for m in (mask, mask[0]):
+        bridge._TREE_CALLS.clear()
         got = bridge.run_tree_sparse_kernel(q, k, v, m, block_m=bm, block_n=bn)
+        assert [e is not False for e in bridge._TREE_CALLS.values()] == [True]
+        assert _tree_call_route(q, k, v, m, bm, bn) == route
         meta = bridge.build_tree_metadata(m, p, bm, bn)
         want = bridge.run_tree_sparse_kernel(q, k, v, None, block_m=bm, block_n=bn, metadata=meta)
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
