@@ -507,7 +507,7 @@ template <int LPU, int K> __device__ inline void wait_units(int k) {
 // The workgroup's dQ^T adds to the fp32 accumulator once at the end
 // (atomics: several splits of one chunk add to the same rows).
 //
-// What bounds it: VALU issue and latency (40 % MFMA busy, 9.5 VALU per MFMA
+// What bounds it: VALU issue and latency (40 % MFMA busy, 10.5 VALU per MFMA
 // at the 1024-token tree behind 16k keys when every unit built and tested a
 // visibility bit per score and the softmax sat between the MFMA groups).  A
 // unit runs S^T; dP^T with the exponentials between its MFMAs; dQ^T's first

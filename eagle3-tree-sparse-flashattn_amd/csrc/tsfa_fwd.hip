@@ -1209,7 +1209,7 @@ void split_kernel(const SplitArgs a) {
     // row_ptr window, then every CSR entry of those rows at once.
     // MASK: the q-blocks' rows packed straight from the mask, one round trip
     // and no builder launch before this kernel (the 8B decode shape's verify
-    // call 17.8 -> 14.9 us); a block with a visible pair marks the units it
+    // call 17.9 -> 15.2 us); a block with a visible pair marks the units it
     // overlaps, so the visited units are the CSR record's.
     auto build_state = [&]() {
       for (int i = tid; i < n_st; i += kWaves * 64) st[i] = 0;
