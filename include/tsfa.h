@@ -169,9 +169,9 @@ int tsfa_fwd_lse(const void* q, const void* k, const void* v, void* o, float* ls
  * tsfa_bwd_workspace_bytes(..., n_trees) bytes, n_trees = batch when
  * meta_seq_stride is non-zero (one tree per sequence), else 1.  Two or
  * three kernel launches on `stream`, no host synchronisation: the dK / dV and
- * dQ workgroups share one launch (TSFA_BWD_CONCURRENT=0: one after the
- * other).  Supported: the
- * shapes tsfa_fwd supports with q_len * gqa_group_size < 2^22; the tree's
+ * dQ workgroups share one launch (TSFA_BWD_CONCURRENT=0, or more of them than
+ * one grid holds: one after the other).  Strides may be negative.  Supported:
+ * the shapes tsfa_fwd supports with q_len * gqa_group_size < 2^22; the tree's
  * block-state table of one 32-row tile must fit 8192 entries (otherwise
  * TSFA_ERR_UNSUPPORTED, as tsfa_bwd_workspace_bytes returning 0 signals). */
 size_t tsfa_bwd_workspace_bytes(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len,
