@@ -2507,6 +2507,10 @@ int fwd_impl(const void* q, const KvSource& kv, void* o, float* lse, const TreeS
                     gqa_group_size, block_m, block_n, head_dim, dtype, workspace, workspace_bytes,
                     reinterpret_cast<hipStream_t>(stream_), q_strides);
 
+  if (!kv.paged()) {
+    st = check_split_rows(kv.k_strides[2], kv.v_strides[2]);
+    if (st != TSFA_OK) return st;
+  }
   // one snapshot of the TSFA_* switches for the whole call
   const Config cfg = config();
   Plan p;

@@ -312,11 +312,16 @@ int check_kv_strides(const void* k, const int64_t* k_strides, const void* v, con
   return TSFA_OK;
 }
 
+int check_split_rows(int64_t k_row_stride, int64_t v_row_stride) {
+  return k_row_stride < 0 || v_row_stride < 0 ? TSFA_ERR_UNSUPPORTED : TSFA_OK;
+}
+
 int check_paged(int batch, int kv_len, const void* cache, const int64_t* cache_strides, const int32_t* kv_indptr,
                 int64_t pt_stride, int64_t n_indices, int n_pages, int page_size) {
   if (cache == nullptr || cache_strides == nullptr) return TSFA_ERR_INVALID_ARGUMENT;
   if (!rows_ok(cache_strides, 5) || !aligned16(cache)) return TSFA_ERR_UNSUPPORTED;
   if (cache_strides[2] >= ((int64_t)1 << 26)) return TSFA_ERR_UNSUPPORTED;  // 32-bit lane offsets
+  if (check_split_rows(cache_strides[2], cache_strides[2]) != TSFA_OK) return TSFA_ERR_UNSUPPORTED;
   // pages of 16 keys or more, a power of two: a wave's 16-key DMA share
   // then spans at most two pages
   if (page_size < 16 || (page_size & (page_size - 1)) != 0) return TSFA_ERR_UNSUPPORTED;

@@ -134,6 +134,9 @@ int check_args(int batch, int num_heads, int num_kv_heads, int q_len, int kv_len
 // cache strides [page, slot, row, head, d].
 int check_strides(const void* q, const int64_t* q_strides, const void* o, const int64_t* o_strides);
 int check_kv_strides(const void* k, const int64_t* k_strides, const void* v, const int64_t* v_strides);
+// K/V rows of the split kernel: its 32-bit lane offsets are unsigned, so a
+// negative row stride is refused (the generic kernel's addresses are 64-bit).
+int check_split_rows(int64_t k_row_stride, int64_t v_row_stride);
 int check_paged(int batch, int kv_len, const void* cache, const int64_t* cache_strides, const int32_t* kv_indptr,
                 int64_t pt_stride, int64_t n_indices, int n_pages, int page_size);
 

@@ -105,7 +105,9 @@ int tsfa_pack_bits_host(const uint8_t* bits, int64_t n_bits, int32_t* words);
  * k, v      [B, Hkv, kv_len, D] of `dtype`, last-dim stride 1
  * strides   int64[16]: q(b,h,n,d), k(b,h,n,d), v(b,h,n,d), o(b,h,n,d) in
  *           elements, the reference's stride arguments in order
- *           (tree_sparse_flashattn.py:174-189); every d stride must be 1
+ *           (tree_sparse_flashattn.py:174-189); every d stride must be 1, and
+ *           16-bit K/V of head_dim 64 or 128 must not step back from key to
+ *           key (TSFA_ERR_UNSUPPORTED; the paged cache's rows likewise)
  * metadata  row_ptr/col_idx/blk_type/payload/offset as produced by
  *           prepare_tree_sparse_metadata; meta_seq_stride[5] gives the
  *           per-batch-element stride (elements) of each of the five arrays:

@@ -207,6 +207,12 @@ static void sweep_layouts() {
     EXPECT(st >= 0 && st <= 2, "paged %d", st);
     (void)fwd::paged_offsets_fit_32((int)uni(-1, 1 << 24), s5[0], s5[2], (int)uni(-1, 512), (int)uni(-1, 256));
   }
+  // keys stored last to first: the split kernel's lane offsets are unsigned
+  const int64_t rev[5] = {16 * 1024, 8 * 1024, -1024, 128, 1}, dense[5] = {16 * 1024, 8 * 1024, 1024, 128, 1};
+  EXPECT(fwd::check_paged(1, 100, al, rev, nullptr, 100, 100, 100, 16) == TSFA_ERR_UNSUPPORTED, "reversed pages");
+  EXPECT(fwd::check_paged(1, 100, al, dense, nullptr, 100, 100, 100, 16) == TSFA_OK, "pages");
+  EXPECT(fwd::check_split_rows(-128, 128) == TSFA_ERR_UNSUPPORTED && fwd::check_split_rows(128, -8) != TSFA_OK &&
+             fwd::check_split_rows(0, 128) == TSFA_OK, "rows");
   // the 32-bit paged kernel: FlashInfer's NHD pool of 1000 pages fits; a
   // permuted [page_size, pages, 2, Hkv, D] pool whose row stride spans every
   // page does not, although pages * page_stride alone would (2048-element

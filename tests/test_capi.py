@@ -158,3 +158,16 @@ def test_tree_attention_rejects_on_the_host():
     assert st == _lib.TSFA_ERR_INVALID_ARGUMENT
     assert lib.tsfa_tree_attention_workspace_bytes(1, 8, 2, 40, 30, 1, 16, 32, 128, 1) == 0
     assert lib.tsfa_tree_attention_workspace_bytes(2, 8, 2, 40, 100, 3, 16, 32, 128, 1) == 0  # n_masks not 1 or B
+
+
+@needs_full_library
+@pytest.mark.parametrize("rows", [(-128, 128), (128, -128)])
+def test_split_kernel_refuses_negative_key_strides(rows):
+    # keys stored last to first: the 16-bit kernel's lane offsets are unsigned
+    # (refused on the host; the pointers are never dereferenced)
+    fake, n = 0x2000, FWD_OK["kv_len"]
+    strides = (ctypes.c_int64 * 16)(*(64 * 32 * 128, 64 * 128, 128, 1), *(8 * n * 128, n * 128, rows[0], 1),
+                                    *(8 * n * 128, n * 128, rows[1], 1), *(64 * 32 * 128, 64 * 128, 128, 1))
+    st = _lib.load().tsfa_fwd(*[fake] * 9, (ctypes.c_int64 * 5)(), strides, ctypes.c_float(0.1), *FWD_OK.values(), fake,
+                              1 << 30, None)
+    assert st == _lib.TSFA_ERR_UNSUPPORTED
